@@ -19,6 +19,9 @@
 //    copy, so an index error reads 0 / drops the atomic instead of faulting;
 //  * the adjoint scatters with buffer float atomics into the same two
 //    layouts, then one pass sums them into the x-fastest output.
+// The exact pair of every geometry without steep rays takes the fan-plane
+// kernels of siddon_fan.h instead; the walks here take the reference rule,
+// the counter and steep rays.
 #include <algorithm>
 #include <type_traits>
 #include <cmath>
@@ -524,6 +527,8 @@ struct Launch {
     int nv;
     unsigned flags;
     float sbound;        // upper bound of any ray's mm per slab (fixed-point adjoint scale)
+    int fan;             // 1: walked on fan planes (siddon_fan.h)
+    const void* cols;    // fan planes: column records of every view, or null
 };
 
 // A helical view's lift: source and detector of view iv raised by zoff[iv]
@@ -1508,6 +1513,8 @@ __global__ __launch_bounds__(64 * NW, 4) void k_siddon_adj_tile(Launch P, const 
                                                  false);
 }
 
+#include "siddon_fan.h"
+
 // Launch of one tile-adjoint variant.
 template <int TX, int TY, int TZ, int NW, int CS>
 void launch_tile(bool ref, bool fix, const Launch& L, const float* pv, float* image, const unsigned* maxbits,
@@ -1529,21 +1536,55 @@ void launch_tile(bool ref, bool fix, const Launch& L, const float* pv, float* im
                            sbound);
 }
 
-// max |x| over n values, as float bits, into *out (which the caller zeroes);
-// NaN compares above Inf in this order
-__global__ __launch_bounds__(256) void k_absmax(const float* __restrict__ x, size_t n, unsigned* __restrict__ out)
+// max |x| of a workgroup's share of n values, as float bits, into *out (which
+// the caller zeroes; NaN compares above Inf in this order), four values per
+// load.  One atomic per workgroup: atomics on one word run one after another
+// (~11 ns each: 16384 of them, one per wavefront, took 188 us).
+constexpr int ABS_T = 1024;         // threads per workgroup
+constexpr int ABS_BLOCKS = 512;     // workgroups: two per CU
+__device__ __forceinline__ void absmax_share(const float* __restrict__ x, size_t n, size_t first, size_t stride,
+                                             unsigned* __restrict__ out)
 {
+    __shared__ unsigned red[ABS_T / 64];
     unsigned m = 0u;
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256)
-        m = max(m, __float_as_uint(x[i]) & 0x7fffffffu);
+    const size_t n4 = n / 4;
+    for (size_t i = first; i < n4; i += stride) {
+        uint4 v;                                    // 4-byte aligned
+        __builtin_memcpy(&v, x + 4 * i, 16);
+        m = max(max(m, v.x & 0x7fffffffu), max(v.y & 0x7fffffffu, max(v.z & 0x7fffffffu, v.w & 0x7fffffffu)));
+    }
+    if (first < n - 4 * n4) m = max(m, __float_as_uint(x[4 * n4 + first]) & 0x7fffffffu);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, o, 64));
-    if ((threadIdx.x & 63) == 0) atomicMax(out, m);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int w = 1; w < ABS_T / 64; ++w) m = max(m, red[w]);
+        if (m) atomicMax(out, m);
+    }
 }
 
-__global__ void k_view_trig(const float* __restrict__ angles, int nv, double* __restrict__ trig)
+// ... of a sinogram; clears nsum words of sums (the adjoint's split sums) on the way
+__global__ __launch_bounds__(ABS_T) void k_absmax(const float* __restrict__ x, size_t n, unsigned* __restrict__ out,
+                                                  unsigned long long* __restrict__ sums, size_t nsum)
+{
+    const size_t first = (size_t)blockIdx.x * ABS_T + threadIdx.x, stride = (size_t)gridDim.x * ABS_T;
+    for (size_t i = first; i < nsum; i += stride) sums[i] = 0ull;
+    absmax_share(x, n, first, stride, out);
+}
+
+inline unsigned absmax_blocks(size_t n)
+{
+    return (unsigned)std::max<size_t>(1, std::min<size_t>(ABS_BLOCKS, n / (8 * ABS_T)));
+}
+
+// (cos, sin) of every view; clears *zero (the max word of a fixed-point adjoint) if given
+__global__ void k_view_trig(const float* __restrict__ angles, int nv, double* __restrict__ trig,
+                            unsigned* __restrict__ zero)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (zero && i == 0) *zero = 0u;
     if (i >= nv) return;
     const double a = (double)angles[i];
     trig[2 * i] = cos(a);
@@ -1717,12 +1758,14 @@ Launch make_launch(const int grid[3], const float center[3], const float size[3]
     L.nv = nv;
     L.flags = flags;
     L.sbound = scale_bound(L.V, L.G, flags);
+    L.fan = fan_ok(L.V, L.G, flags) ? 1 : 0;
+    L.cols = nullptr;
     return L;
 }
 
-void launch_trig(const float* angles, int nv, double* trig, hipStream_t st)
+void launch_trig(const float* angles, int nv, double* trig, hipStream_t st, unsigned* zero = nullptr)
 {
-    hipLaunchKernelGGL(k_view_trig, dim3((nv + 255) / 256), dim3(256), 0, st, angles, nv, trig);
+    hipLaunchKernelGGL(k_view_trig, dim3((nv + 255) / 256), dim3(256), 0, st, angles, nv, trig, zero);
 }
 
 void launch_pad(const float* image, const int grid[3], const WsPlan& p, char* ws, hipStream_t st)
@@ -1756,6 +1799,15 @@ int run_forward(const float* image, const int grid[3], const float center[3], co
     hipStream_t s = (hipStream_t)stream;
     char* ws = (char*)workspace;
     Launch L = make_launch(grid, center, size, nv, SID, SAD, na, da, ai, nb, db, bi, cyl, flags, ws, p, zoff);
+    if (L.fan) {
+        // the z-fastest copy fits the space of the two padded copies
+        launch_fan_prep(image, grid, L.Ly.xf, angles, nv, (double*)(ws + p.trig_off), s);
+        const size_t cols_off = p.xf_off + align256(sizeof(float) * (size_t)grid[0] * grid[1] * fan_row(grid[2]));
+        if (cols_off < p.total) launch_fan_cols(L, ws + cols_off, p.total - cols_off, s);
+        launch_fan_fwd(L, out, fwd_vg_log2(flags, nv), s);
+        NEFCT_CHECK_LAUNCH();
+        return NEFCT_OK;
+    }
     launch_trig(angles, nv, (double*)(ws + p.trig_off), s);
     launch_pad(image, grid, p, ws, s);
     if (flags & NEFCT_F_REF_SLAB)
@@ -1766,7 +1818,8 @@ int run_forward(const float* image, const int grid[3], const float center[3], co
     return NEFCT_OK;
 }
 
-void launch_adjoint_tiles(const Launch& L, const float* pv, float* image, unsigned* maxbits, hipStream_t s);
+void launch_adjoint_tiles(Launch& L, const float* pv, float* image, unsigned* maxbits, char* room, size_t bytes,
+                          hipStream_t s);
 
 int run_adjoint(const float* pv, const int grid[3], const float center[3], const float size[3], const float* angles,
                 int nv, float SID, float SAD, int na, float da, float ai, int nb, float db, float bi, int cyl,
@@ -1781,11 +1834,13 @@ int run_adjoint(const float* pv, const int grid[3], const float center[3], const
     hipStream_t s = (hipStream_t)stream;
     char* ws = (char*)workspace;
     Launch L = make_launch(grid, center, size, nv, SID, SAD, na, da, ai, nb, db, bi, cyl, flags, ws, p, zoff);
-    launch_trig(angles, nv, (double*)(ws + p.trig_off), s);
     const int nx = grid[0], ny = grid[1], nz = grid[2];
     const bool ref = (flags & NEFCT_F_REF_SLAB) != 0;
-    if (flags & NEFCT_F_ADJ_WINDOW) {
-        // ray tiles with LDS slab windows flushed by global atomics
+    unsigned* maxbits = (unsigned*)(ws + p.xf_off);
+    launch_trig(angles, nv, (double*)(ws + p.trig_off), s, maxbits);
+    if ((flags & NEFCT_F_ADJ_WINDOW) && !L.fan) {
+        // ray tiles with LDS slab windows flushed by global atomics (rays on
+        // fan planes take the float variant of their own adjoint instead)
         launch_zero((float*)(ws + p.xf_off), p.xf_elems, s);
         launch_zero((float*)(ws + p.yf_off), p.yf_elems, s);
         const dim3 g((na + BX - 1) / BX, (nb + BY * AR - 1) / (BY * AR), nv), b(BX, BY);
@@ -1797,9 +1852,10 @@ int run_adjoint(const float* pv, const int grid[3], const float center[3], const
                            (const float*)(ws + p.xf_off), (const float*)(ws + p.yf_off), nx, ny, nz, p.NXP, p.NYP,
                            image);
     } else {
-        // the max |projection| word goes to the otherwise unused padded-copy
-        // region of the workspace
-        launch_adjoint_tiles(L, pv, image, (unsigned*)(ws + p.xf_off), s);
+        // the max |projection| word, a split's sums and the column records go
+        // to the otherwise unused padded-copy region of the workspace
+        const size_t off = p.xf_off + 256;
+        launch_adjoint_tiles(L, pv, image, maxbits, ws + off, p.total > off ? p.total - off : 0, s);
     }
     NEFCT_CHECK_LAUNCH();
     return NEFCT_OK;
@@ -1807,18 +1863,34 @@ int run_adjoint(const float* pv, const int grid[3], const float center[3], const
 
 // The volume-tile adjoint (every variant but the slab windows): volume blocks
 // own their voxels.  L.trig must hold the view table.  Fixed-point
-// accumulation first needs max |projection|, into *maxbits (cleared here).
-void launch_adjoint_tiles(const Launch& L, const float* pv, float* image, unsigned* maxbits, hipStream_t s)
+// accumulation first needs max |projection|, into *maxbits (cleared by the
+// caller).  room: scratch of `bytes` bytes (256-byte aligned) or null; used for
+// a split's sums (8 bytes per voxel) and the column records where they fit.
+void launch_adjoint_tiles(Launch& L, const float* pv, float* image, unsigned* maxbits, char* room, size_t bytes,
+                          hipStream_t s)
 {
     const unsigned flags = L.flags;
     const bool ref = (flags & NEFCT_F_REF_SLAB) != 0;
     {
-        const bool fix = !(flags & NEFCT_F_ADJ_FLOAT_ATOMIC);
+        const bool fix = !(flags & (NEFCT_F_ADJ_FLOAT_ATOMIC | NEFCT_F_ADJ_WINDOW));
+        int nsplit = 1;
+        unsigned long long* sums = (unsigned long long*)room;
+        if (L.fan) {
+            const size_t vol = align256(sizeof(unsigned long long) * (size_t)L.V.n[0] * L.V.n[1] * L.V.n[2]);
+            const long long blocks = (long long)((L.V.n[0] + FB - 1) / FB) * ((L.V.n[1] + FB - 1) / FB) *
+                                     fan_zblocks(L.V.n[2], FAN_TZ);
+            if (fix && room && vol <= bytes) nsplit = fan_splits(blocks, L.nv);
+            const size_t used = nsplit > 1 ? vol : 0;
+            launch_fan_cols(L, room ? room + used : nullptr, bytes - used, s);
+        }
         if (fix) {
             const size_t n = (size_t)L.nv * (size_t)L.G.na * (size_t)L.G.nb;
-            launch_zero((float*)maxbits, 1, s);
-            const size_t blocks = std::min<size_t>(4096, (n + 255) / 256);
-            hipLaunchKernelGGL(k_absmax, dim3((unsigned)blocks), dim3(256), 0, s, pv, n, maxbits);
+            hipLaunchKernelGGL(k_absmax, dim3(absmax_blocks(n)), dim3(ABS_T), 0, s, pv, n, maxbits, sums,
+                               nsplit > 1 ? (size_t)L.V.n[0] * L.V.n[1] * L.V.n[2] : (size_t)0);
+        }
+        if (L.fan) {
+            launch_fan_adj(L, pv, image, sums, nsplit, maxbits, s);
+            return;
         }
         const float sb = L.sbound;
         const unsigned shape = flags & NEFCT_F_TILE_MASK;
@@ -1886,6 +1958,8 @@ __device__ Launch launch_of(const nefct_problem& pr, char* ws_base, unsigned fla
     L.nv = pr.nv;
     L.flags = flags;
     L.sbound = scale_bound(L.V, L.G, flags);
+    L.fan = fan_ok(L.V, L.G, flags) ? 1 : 0;
+    L.cols = nullptr;
     return L;
 }
 
@@ -1913,14 +1987,24 @@ __host__ __device__ inline size_t batch_max_off(int nprob) { return Q_HEADER + b
 __host__ __device__ inline size_t batch_head_bytes(int nprob) { return batch_max_off(nprob) + align256(4 * (size_t)nprob); }
 
 // trig tables and launch parameters of every problem; zeroed max words
-__global__ void k_batch_prep(const nefct_problem* __restrict__ probs, int nprob, char* ws_base, unsigned flags)
+// cols: 1 in a forward (the column records follow the volume's copy), 2 in an
+// adjoint (they take its place)
+__global__ void k_batch_prep(const nefct_problem* __restrict__ probs, int nprob, char* ws_base, unsigned flags,
+                             int cols)
 {
     const int p = blockIdx.y;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= nprob) return;
     const nefct_problem& pr = probs[p];
     if (i == 0) {
-        ((Launch*)(ws_base + Q_HEADER))[p] = launch_of(pr, ws_base, flags);
+        Launch L = launch_of(pr, ws_base, flags);
+        if (pr.pad_) {
+            const WsPlan w = plan_ws(pr.grid, pr.nv);
+            const size_t off = w.xf_off + (cols == 1 ? align256(sizeof(float) * (size_t)pr.grid[0] * pr.grid[1] *
+                                                                fan_row(pr.grid[2])) : 0);
+            if (off + sizeof(FanCol) * (size_t)pr.na * (size_t)pr.nv <= w.total) L.cols = ws_base + pr.ws_offset + off;
+        }
+        ((Launch*)(ws_base + Q_HEADER))[p] = L;
         ((unsigned*)(ws_base + batch_max_off(nprob)))[p] = 0u;
     }
     if (i >= pr.nv) return;
@@ -1929,6 +2013,24 @@ __global__ void k_batch_prep(const nefct_problem* __restrict__ probs, int nprob,
     const double a = (double)pr.angles[i];
     trig[2 * i] = cos(a);
     trig[2 * i + 1] = sin(a);
+}
+
+// View and ray tile of task id of problem p (see k_batch_fwd).
+__device__ __forceinline__ void batch_fwd_task(const nefct_problem* __restrict__ probs, int nprob, int p,
+                                               long long id, long long total, int& iv, int& ta, int& tb)
+{
+    const nefct_problem& pr = probs[p];
+    const long long begin = pr.tile_begin;
+    const long long n = (p + 1 < nprob ? probs[p + 1].tile_begin : total) - begin;
+    const long long lid = id - begin;
+    const long long local = (lid & 7) * (n >> 3) + (lid >> 3);
+    const unsigned tiles = (unsigned)pr.tiles_a * (unsigned)pr.tiles_b;
+    const unsigned vin = (unsigned)(local % FWD_VG);
+    const long long rest = local / FWD_VG;
+    const unsigned tile = (unsigned)(rest % tiles);
+    iv = (int)((rest / tiles) * FWD_VG + vin);
+    ta = (int)(tile % (unsigned)pr.tiles_a);
+    tb = (int)(tile / (unsigned)pr.tiles_a);
 }
 
 // Forward of every problem in one launch.  Each problem's tasks are numbered
@@ -1940,6 +2042,8 @@ __global__ void k_batch_prep(const nefct_problem* __restrict__ probs, int nprob,
 // eighth of its tasks: all XCDs work on the same problem at a time (one
 // volume in the shared cache, as in one plain call), each on its own views.
 // t0 (a multiple of 8) offsets the chunk this launch covers.
+// Problems walked on fan planes (pad_ = 1) are k_batch_fan_fwd's: their tiles
+// are counted by its own tile size.
 template <bool REF>
 __global__ __launch_bounds__(FX * FY) void k_batch_fwd(const nefct_problem* __restrict__ probs, int nprob,
                                                        long long t0, long long total, char* ws_base)
@@ -1948,36 +2052,55 @@ __global__ __launch_bounds__(FX * FY) void k_batch_fwd(const nefct_problem* __re
     if (id >= total) return;
     const int p = __builtin_amdgcn_readfirstlane(find_problem(probs, nprob, id, false));
     const nefct_problem& pr = probs[p];
-    const long long begin = pr.tile_begin;
-    const long long n = (p + 1 < nprob ? probs[p + 1].tile_begin : total) - begin;
-    const long long lid = id - begin;
-    const long long local = (lid & 7) * (n >> 3) + (lid >> 3);
-    const unsigned tiles = (unsigned)pr.tiles_a * (unsigned)pr.tiles_b;
-    const unsigned vin = (unsigned)(local % FWD_VG);
-    const long long rest = local / FWD_VG;
-    const unsigned tile = (unsigned)(rest % tiles);
-    const int iv = (int)((rest / tiles) * FWD_VG + vin);
+    if (pr.pad_) return;
+    int iv, ta, tb;
+    batch_fwd_task(probs, nprob, p, id, total, iv, ta, tb);
     if (iv >= pr.nv) return;
-    const int ta = (int)(tile % (unsigned)pr.tiles_a), tb = (int)(tile / (unsigned)pr.tiles_a);
     const Launch& L = batch_launches(ws_base)[p];
     siddon_rays<0, REF>(L, ta * FX + threadIdx.x, tb * FY + threadIdx.y, iv, nullptr, pr.sinogram, nullptr);
 }
 
+// k_batch_fwd for the problems walked on fan planes
+__global__ __launch_bounds__(64 * FAN_FW, 8) void k_batch_fan_fwd(const nefct_problem* __restrict__ probs, int nprob,
+                                                              long long t0, long long total, char* ws_base)
+{
+    __shared__ FanSeg tabs[FAN_FW][FAN_TAB];
+    const long long id = t0 + blockIdx.x;
+    if (id >= total) return;
+    const int p = __builtin_amdgcn_readfirstlane(find_problem(probs, nprob, id, false));
+    const nefct_problem& pr = probs[p];
+    if (!pr.pad_) return;
+    int iv, ta, tb;
+    batch_fwd_task(probs, nprob, p, id, total, iv, ta, tb);
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ia = __builtin_amdgcn_readfirstlane(ta * FAN_FW + wv);
+    if (iv >= pr.nv || ia >= pr.na) return;
+    // a copy (in scalar registers: it is never indexed at run time here), so
+    // that stores to the sinogram do not make its fields be read again
+    const Launch L = batch_launches(ws_base)[p];
+    fan_forward_wave(L, ia, tb * 64, iv, tabs[wv], pr.sinogram);
+}
+
+// column records of every fan-plane problem (blockIdx.z = problem, .y = view)
+__global__ __launch_bounds__(256) void k_batch_fan_cols(int nprob, char* ws_base)
+{
+    const int p = blockIdx.z;
+    const Launch& L = batch_launches(ws_base)[p];
+    const int ia = blockIdx.x * 256 + threadIdx.x, iv = blockIdx.y;
+    if (!L.cols || iv >= L.nv || ia >= L.G.na) return;
+    ((FanCol*)L.cols)[(size_t)iv * L.G.na + ia] = fan_column(L.V, L.G, L.trig[2 * iv], L.trig[2 * iv + 1], ia);
+}
+
 // max |sinogram| of every problem (blockIdx.y = problem)
-__global__ __launch_bounds__(256) void k_batch_absmax(const nefct_problem* __restrict__ probs, int nprob,
+__global__ __launch_bounds__(ABS_T) void k_batch_absmax(const nefct_problem* __restrict__ probs, int nprob,
                                                       char* ws_base)
 {
     const int p = blockIdx.y;
     if (p >= nprob) return;
     const nefct_problem& pr = probs[p];
     const size_t n = (size_t)pr.nv * (size_t)pr.na * (size_t)pr.nb;
-    const float* x = pr.sinogram;
-    unsigned m = 0u;
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256)
-        m = max(m, __float_as_uint(x[i]) & 0x7fffffffu);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, o, 64));
-    if ((threadIdx.x & 63) == 0) atomicMax((unsigned*)(ws_base + batch_max_off(nprob)) + p, m);
+    absmax_share(pr.sinogram, n, (size_t)blockIdx.x * ABS_T + threadIdx.x, (size_t)gridDim.x * ABS_T,
+                 (unsigned*)(ws_base + batch_max_off(nprob)) + p);
 }
 
 // One launch over the voxel blocks of every problem: workgroup g takes global
@@ -1995,6 +2118,7 @@ __global__ __launch_bounds__(64 * BNW) void k_batch_adj(const nefct_problem* __r
     if (t >= total) return;
     const int p = __builtin_amdgcn_readfirstlane(find_problem(probs, nprob, t, true));
     const nefct_problem& pr = probs[p];
+    if (pr.pad_) return;        // k_batch_fan_adj's
     // block coordinates made scalar: in vector registers they would carry the
     // block bounds and their derived values into VGPRs
     const int local = __builtin_amdgcn_readfirstlane((int)(t - pr.block_begin));
@@ -2005,6 +2129,29 @@ __global__ __launch_bounds__(64 * BNW) void k_batch_adj(const nefct_problem* __r
     const int es = fixed_exp(((const unsigned*)(ws_base + batch_max_off(nprob)))[p], L.sbound);
     adj_tile_block<REF, true, BTX, BTY, BTZ, BNW, CS>(L, pr.sinogram, const_cast<float*>(pr.volume), bx, by, bz, acc,
                                                      shadows, es, false);
+}
+
+// k_batch_adj for the problems walked on fan planes
+__global__ __launch_bounds__(64 * FAN_NW, 4) void k_batch_fan_adj(const nefct_problem* __restrict__ probs, int nprob,
+                                                                 long long total, char* ws_base)
+{
+    __shared__ FanAcc<FAN_TZ, acc_t<true>> acc;
+    __shared__ FanSeg tabs[FAN_NW][4][FAN_ENT];
+    __shared__ int4 shadows[SHV];
+    __shared__ int2 deals[SHV];
+    const long long t = (long long)blockIdx.x + 65536ll * (long long)blockIdx.y;
+    if (t >= total) return;
+    const int p = __builtin_amdgcn_readfirstlane(find_problem(probs, nprob, t, true));
+    const nefct_problem& pr = probs[p];
+    if (!pr.pad_) return;
+    const int local = __builtin_amdgcn_readfirstlane((int)(t - pr.block_begin));
+    const int bx = __builtin_amdgcn_readfirstlane(local % pr.blocks[0]);
+    const int by = __builtin_amdgcn_readfirstlane((local / pr.blocks[0]) % pr.blocks[1]);
+    const int bz = __builtin_amdgcn_readfirstlane(local / (pr.blocks[0] * pr.blocks[1]));
+    const Launch L = batch_launches(ws_base)[p];
+    const int es = fixed_exp(((const unsigned*)(ws_base + batch_max_off(nprob)))[p], L.sbound);
+    fan_adjoint_block<true, FAN_TZ, FAN_NW>(L, pr.sinogram, const_cast<float*>(pr.volume), nullptr, bx, by, bz,
+                                            pr.blocks[2], 0, pr.nv, acc, tabs, shadows, deals, es);
 }
 
 }  // namespace
@@ -2070,8 +2217,8 @@ int run_adjoint_noalloc(const float* pv, const int grid[3], const float center[3
     p.xf_elems = p.yf_elems = 0;
     Launch L = make_launch(grid, center, size, nv, SID, SAD, na, da, ai, nb, db, bi, cyl, flags, sc, p);
     hipStream_t s = (hipStream_t)stream;
-    launch_trig(angles, nv, (double*)(sc + NOALLOC_TRIG_OFF), s);
-    launch_adjoint_tiles(L, pv, image, (unsigned*)sc, s);
+    launch_trig(angles, nv, (double*)(sc + NOALLOC_TRIG_OFF), s, (unsigned*)sc);
+    launch_adjoint_tiles(L, pv, image, (unsigned*)sc, nullptr, 0, s);
     NEFCT_CHECK_LAUNCH();
     return NEFCT_OK;
 }
@@ -2187,6 +2334,39 @@ int nefct_siddon_count(const int grid[3], const float center[3], const float siz
     return NEFCT_OK;
 }
 
+// Whether a problem's rays are walked on fan planes (its tasks are counted accordingly).
+static bool plan_is_fan(const nefct_problem& pr, unsigned flags)
+{
+    VolDev V;
+    DetDev G;
+    for (int i = 0; i < 3; ++i) {
+        V.n[i] = pr.grid[i];
+        V.vs[i] = (double)pr.size[i] / pr.grid[i];
+        V.inv_vs[i] = 1.0 / V.vs[i];
+    }
+    G.sad = pr.SAD;
+    G.na = pr.na;
+    G.nb = pr.nb;
+    G.db = pr.db;
+    G.bi = pr.bi;
+    return fan_ok(V, G, flags);
+}
+
+// How the batch was planned, against the flags of this call.
+struct BatchKinds {
+    bool fan = false, plain = false, mismatch = false;
+};
+
+static BatchKinds batch_kinds(const nefct_problem* host, int nprob, unsigned flags)
+{
+    BatchKinds k;
+    for (int i = 0; i < nprob; ++i) {
+        (host[i].pad_ ? k.fan : k.plain) = true;
+        if (host[i].pad_ && !plan_is_fan(host[i], flags)) k.mismatch = true;
+    }
+    return k;
+}
+
 int nefct_batch_plan(nefct_problem* probs, int nprob, unsigned flags, size_t* workspace_bytes, long long* total_tiles,
                      long long* total_blocks)
 {
@@ -2200,18 +2380,19 @@ int nefct_batch_plan(nefct_problem* probs, int nprob, unsigned flags, size_t* wo
                           pr.ai, pr.bi, flags);
         if (st) return st;
         if (!pr.volume || !pr.sinogram) return NEFCT_ERR_NULL;
-        pr.tiles_a = (pr.na + FX - 1) / FX;
-        pr.tiles_b = (pr.nb + FY - 1) / FY;
+        const bool fan = plan_is_fan(pr, flags);
+        pr.pad_ = fan ? 1 : 0;
+        pr.tiles_a = fan ? (pr.na + FAN_FW - 1) / FAN_FW : (pr.na + FX - 1) / FX;
+        pr.tiles_b = fan ? (pr.nb + 63) / 64 : (pr.nb + FY - 1) / FY;
         pr.tile_begin = tiles;
         tiles += (long long)pr.tiles_a * pr.tiles_b * ((pr.nv + FWD_VG - 1) / FWD_VG * FWD_VG);
-        pr.blocks[0] = (pr.grid[0] + BTX - 1) / BTX;
-        pr.blocks[1] = (pr.grid[1] + BTY - 1) / BTY;
-        pr.blocks[2] = (pr.grid[2] + BTZ - 1) / BTZ;
+        pr.blocks[0] = fan ? (pr.grid[0] + FB - 1) / FB : (pr.grid[0] + BTX - 1) / BTX;
+        pr.blocks[1] = fan ? (pr.grid[1] + FB - 1) / FB : (pr.grid[1] + BTY - 1) / BTY;
+        pr.blocks[2] = fan ? fan_zblocks(pr.grid[2], FAN_TZ) : (pr.grid[2] + BTZ - 1) / BTZ;
         pr.block_begin = blocks;
         blocks += (long long)pr.blocks[0] * pr.blocks[1] * pr.blocks[2];
         pr.ws_offset = (long long)off;
         off += align256(plan_ws(pr.grid, pr.nv).total);
-        pr.pad_ = 0;
     }
     *workspace_bytes = off;
     *total_tiles = tiles;
@@ -2220,12 +2401,23 @@ int nefct_batch_plan(nefct_problem* probs, int nprob, unsigned flags, size_t* wo
 }
 
 static int batch_prep(const nefct_problem* host, const nefct_problem* dev, int nprob, char* ws, unsigned flags,
-                      hipStream_t s)
+                      int cols, hipStream_t s)
 {
     int maxnv = 1;
     for (int i = 0; i < nprob; ++i) maxnv = max(maxnv, host[i].nv);
-    hipLaunchKernelGGL(k_batch_prep, dim3((maxnv + 255) / 256, nprob), dim3(256), 0, s, dev, nprob, ws, flags);
+    hipLaunchKernelGGL(k_batch_prep, dim3((maxnv + 255) / 256, nprob), dim3(256), 0, s, dev, nprob, ws, flags, cols);
     return NEFCT_OK;
+}
+
+// column records of the fan-plane problems, after batch_prep
+static void batch_cols(const nefct_problem* host, int nprob, char* ws, hipStream_t s)
+{
+    int maxnv = 1, maxna = 1;
+    for (int i = 0; i < nprob; ++i) {
+        maxnv = std::max(maxnv, host[i].nv);
+        maxna = std::max(maxna, host[i].na);
+    }
+    hipLaunchKernelGGL(k_batch_fan_cols, dim3((maxna + 255) / 256, maxnv, nprob), dim3(256), 0, s, nprob, ws);
 }
 
 int nefct_batch_project(const nefct_problem* host, const nefct_problem* dev, int nprob, long long total_tiles,
@@ -2238,15 +2430,35 @@ int nefct_batch_project(const nefct_problem* host, const nefct_problem* dev, int
         return NEFCT_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
     char* ws = (char*)workspace;
-    batch_prep(host, dev, nprob, ws, flags, s);
+    const BatchKinds kinds = batch_kinds(host, nprob, flags);
+    if (kinds.mismatch) {       // planned for the exact rule, called with the reference's: one by one
+        for (int i = 0; i < nprob; ++i) {
+            const nefct_problem& q = host[i];
+            const int st = run_forward(q.volume, q.grid, q.center, q.size, q.angles, q.nv, q.SID, q.SAD, q.na, q.da,
+                                       q.ai, q.nb, q.db, q.bi, q.cyl, q.sinogram, flags, ws + q.ws_offset,
+                                       plan_ws(q.grid, q.nv).total, stream);
+            if (st) return st;
+        }
+        return NEFCT_OK;
+    }
+    batch_prep(host, dev, nprob, ws, flags, 1, s);
     for (int i = 0; i < nprob; ++i) {
         const WsPlan p = plan_ws(host[i].grid, host[i].nv);
-        launch_pad(host[i].volume, host[i].grid, p, ws + host[i].ws_offset, s);
+        char* w = ws + host[i].ws_offset;
+        if (host[i].pad_)
+            launch_fan_prep(host[i].volume, host[i].grid, (float*)(w + p.xf_off), nullptr, 0, nullptr, s);
+        else
+            launch_pad(host[i].volume, host[i].grid, p, w, s);
     }
+    if (kinds.fan) batch_cols(host, nprob, ws, s);
     // chunks of at most 2^31 / 256 workgroups (1-D grid of 32-bit work-items)
     const long long chunk = (0x7fffffffll / (FX * FY)) / 8 * 8;
     for (long long t0 = 0; t0 < total_tiles; t0 += chunk) {
         const long long blocks = std::min(chunk, total_tiles - t0);
+        if (kinds.fan)
+            hipLaunchKernelGGL(k_batch_fan_fwd, dim3((unsigned)blocks), dim3(64 * FAN_FW), 0, s, dev, nprob, t0,
+                               total_tiles, ws);
+        if (!kinds.plain) continue;
         if (flags & NEFCT_F_REF_SLAB)
             hipLaunchKernelGGL((k_batch_fwd<true>), dim3((unsigned)blocks), dim3(FX, FY), 0, s, dev, nprob, t0,
                                total_tiles, ws);
@@ -2268,17 +2480,37 @@ int nefct_batch_backproject(const nefct_problem* host, const nefct_problem* dev,
         return NEFCT_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
     char* ws = (char*)workspace;
-    batch_prep(host, dev, nprob, ws, flags, s);
+    const BatchKinds kinds = batch_kinds(host, nprob, flags);
+    if (kinds.mismatch) {
+        // (the launch-shape flags that the batch does not know are dropped, as below)
+        const unsigned fl = flags & ~(NEFCT_F_ADJ_FLOAT_ATOMIC | NEFCT_F_ADJ_WINDOW | NEFCT_F_DETERMINISTIC);
+        for (int i = 0; i < nprob; ++i) {
+            const nefct_problem& q = host[i];
+            const int st = run_adjoint(q.sinogram, q.grid, q.center, q.size, q.angles, q.nv, q.SID, q.SAD, q.na, q.da,
+                                       q.ai, q.nb, q.db, q.bi, q.cyl, const_cast<float*>(q.volume), fl,
+                                       ws + q.ws_offset, plan_ws(q.grid, q.nv).total, stream);
+            if (st) return st;
+        }
+        return NEFCT_OK;
+    }
+    batch_prep(host, dev, nprob, ws, flags, 2, s);
+    if (kinds.fan) batch_cols(host, nprob, ws, s);
     size_t maxn = 1;
     for (int i = 0; i < nprob; ++i)
         maxn = std::max(maxn, (size_t)host[i].nv * (size_t)host[i].na * (size_t)host[i].nb);
-    const unsigned bx = (unsigned)std::min<size_t>(1024, (maxn + 255) / 256);
-    hipLaunchKernelGGL(k_batch_absmax, dim3(bx, nprob), dim3(256), 0, s, dev, nprob, ws);
+    const unsigned bx = std::min<unsigned>(absmax_blocks(maxn), nprob >= 8 ? 64u : (unsigned)ABS_BLOCKS);
+    hipLaunchKernelGGL(k_batch_absmax, dim3(bx, nprob), dim3(ABS_T), 0, s, dev, nprob, ws);
     if (total_blocks <= 0) return NEFCT_OK;
     if (total_blocks > 65536ll * 65535ll) return NEFCT_ERR_SHAPE;
     const dim3 g((unsigned)std::min<long long>(total_blocks, 65536), (unsigned)((total_blocks + 65535) / 65536));
     // lanes one or two detector rows apart (NEFCT_F_LANE_STRIDE2), as in the plain adjoint
     const bool cs2 = (flags & NEFCT_F_LANE_STRIDE2) != 0;
+    if (kinds.fan)
+        hipLaunchKernelGGL(k_batch_fan_adj, g, dim3(64 * FAN_NW), 0, s, dev, nprob, total_blocks, ws);
+    if (!kinds.plain) {
+        NEFCT_CHECK_LAUNCH();
+        return NEFCT_OK;
+    }
     if (flags & NEFCT_F_REF_SLAB) {
         if (cs2)
             hipLaunchKernelGGL((k_batch_adj<true, 2>), g, dim3(64 * BNW), 0, s, dev, nprob, total_blocks, ws, flags);

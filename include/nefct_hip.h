@@ -64,7 +64,11 @@ typedef enum {
  *                             (fixed order); without: no change (already so)
  *   NEFCT_F_ADJ_WINDOW        ray tiles with LDS slab windows flushed by global
  *                             float atomics
- * A non-finite projection value makes the fixed-point result NaN. */
+ * A non-finite projection value makes the fixed-point result NaN.
+ * The exact rule on geometries whose rays step at most one z cell per slab has
+ * kernels of its own, whose blocks and ray tiles are fixed: there the shape,
+ * lane spacing and forward tile bits below change nothing, and ADJ_WINDOW
+ * means FLOAT_ATOMIC. */
 #define NEFCT_F_DETERMINISTIC 16u
 #define NEFCT_F_ADJ_WINDOW 32u
 #define NEFCT_F_ADJ_FLOAT_ATOMIC 0x1000u
@@ -201,12 +205,12 @@ typedef struct {
     int na, nb;
     float da, ai, db, bi;
     /* filled by nefct_batch_plan */
-    long long tile_begin;   /* first forward task (16x16 rays of one view; views padded to groups of 16) */
-    long long block_begin;  /* first adjoint task (one 32x32x16 voxel block) */
+    long long tile_begin;   /* first forward task (one ray tile of one view; views padded to groups of 16) */
+    long long block_begin;  /* first adjoint task (one voxel block) */
     long long ws_offset;    /* byte offset of the problem's workspace region */
     int tiles_a, tiles_b;
     int blocks[3];
-    int pad_;
+    int pad_;            /* work mapping chosen by nefct_batch_plan */
 } nefct_problem;
 
 /* Validates the problems, fills their plan fields and returns the workspace
@@ -222,7 +226,8 @@ int nefct_batch_project(const nefct_problem* host_problems, const nefct_problem*
                         long long total_tiles, unsigned flags, void* workspace, size_t workspace_bytes, void* stream);
 
 /* Exact (or reference-mode) adjoint of every problem: one max-|projection|
- * pass, then one launch with a workgroup per 32x32x16 voxel block.  Every
+ * pass, then one launch with a workgroup per voxel block (16x16x52 at most, 32x32x16 with
+ * the reference rule or steep rays).  Every
  * output volume is fully written.  NEFCT_F_LANE_STRIDE2 spaces a wavefront's
  * lanes two detector rows apart, as in the plain adjoint (identical result);
  * the other launch-shape flags do not apply to the batched kernels. */
