@@ -809,49 +809,10 @@ __global__ __launch_bounds__(64 * NW, 4) void k_fan_adj(Launch P, const float* _
                                    deals, es);
 }
 
-// Voxels from the integer sums of several view ranges.
-__global__ __launch_bounds__(256) void k_fan_sums(const unsigned long long* __restrict__ sums, size_t n,
-                                                  const unsigned* __restrict__ maxbits, float sbound,
-                                                  float* __restrict__ image)
-{
-    const int es = fixed_exp(*maxbits, sbound);
-    const bool poisoned = es == FIX_POISON;
-    const double inv_s = poisoned ? 1.0 : ldexp(1.0, -es);
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
-        if (poisoned)
-            reinterpret_cast<unsigned*>(image)[i] = 0x7fc00000u;
-        else
-            image[i] = (float)((double)(long long)sums[i] * inv_s);
-    }
-}
-
 constexpr int FAN_TZ = 52;      // tallest block of the fixed-point and float adjoints
 constexpr int FAN_NW = 16;
 
-// Number of view ranges a block's work is split into.  A workgroup fills a
-// CU, so few blocks leave CUs idle (32 blocks at 64^3) or a last round nearly
-// empty; the ranges' integer sums are added in the workspace (8 B per voxel
-// and range through the L2) and need at least 8 views each to be worth it.
-// The smallest split whose last round leaves 10 % fewer CUs idle: 64^3 voxels,
-// 128^2 cells, 120 views 2226 -> 135 us (1854 us of it the whole adjoint on
-// 16 CUs, 188 us the maximum's atomics).
-inline int fan_splits(long long blocks, int nv)
-{
-    constexpr int CUS = 256;
-    int best = 1;
-    double eff = 0.0;
-    for (int ns = 1; ns <= 64 && (ns == 1 || nv / ns >= 8); ++ns) {
-        const long long w = blocks * ns, rounds = (w + CUS - 1) / CUS;
-        const double e = (double)w / (double)(rounds * CUS);
-        if (e > eff + 0.1) {
-            eff = e;
-            best = ns;
-        }
-    }
-    return best;
-}
-
-// sums: 8 bytes per voxel of scratch (cleared by launch_absmax), or null
+// sums: a split's scratch (cleared by k_absmax), or null without one
 void launch_fan_adj(const Launch& L, const float* pv, float* image, unsigned long long* sums, int nsplit,
                     const unsigned* maxbits, hipStream_t s)
 {
@@ -866,10 +827,6 @@ void launch_fan_adj(const Launch& L, const float* pv, float* image, unsigned lon
         return;
     }
     hipLaunchKernelGGL((k_fan_adj<true, FAN_TZ, FAN_NW>), g, dim3(64 * FAN_NW), 0, s, L, pv, image,
-                       nsplit > 1 ? sums : nullptr, nsplit, maxbits);
-    if (nsplit > 1) {
-        const size_t n = (size_t)L.V.n[0] * L.V.n[1] * L.V.n[2];
-        hipLaunchKernelGGL(k_fan_sums, dim3((unsigned)std::min<size_t>(2048, (n + 255) / 256)), dim3(256), 0, s, sums,
-                           n, maxbits, L.sbound, image);
-    }
+                       sums, nsplit, maxbits);
+    if (sums) launch_split_sums(L, sums, maxbits, image, s);
 }
