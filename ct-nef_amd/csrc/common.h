@@ -22,6 +22,48 @@ __device__ __forceinline__ float buf_load(__amdgpu_buffer_rsrc_t r, int byte_off
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, byte_off, 0, 0));
 }
 
+// four floats from a byte offset that is a multiple of 4
+__device__ __forceinline__ float4 buf_load4(__amdgpu_buffer_rsrc_t r, int byte_off)
+{
+    return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, byte_off, 0, 0));
+}
+
+// One dword per lane from byte offset lane_off + off of a raw buffer straight
+// into LDS at lds + 4 lane (no registers; past the buffer's end: 0).  All of
+// off, lds and the buffer are wave-uniform and every lane is active.  Written
+// as assembly because the compiler holds back every later LDS read until such
+// loads have landed: the caller waits with lds_loads_done() before the barrier
+// that hands the cells over.
+typedef int rsrc_words __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ rsrc_words make_rsrc_words(const void* p, uint32_t nbytes)
+{
+    const uint64_t a = (uint64_t)p;
+    rsrc_words r;
+    r.x = __builtin_amdgcn_readfirstlane((int)(uint32_t)a);
+    r.y = __builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32) & 0xffff);
+    r.z = __builtin_amdgcn_readfirstlane((int)nbytes);
+    r.w = 0x00020000;
+    return r;
+}
+
+__device__ __forceinline__ void buf_load_lds(rsrc_words r, int lane_off, unsigned off, unsigned lds)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
+                 :
+                 : "s"(__builtin_amdgcn_readfirstlane((int)lds)), "v"(lane_off), "s"(r),
+                   "s"(__builtin_amdgcn_readfirstlane((int)off))
+                 : "memory");
+#endif
+}
+
+__device__ __forceinline__ void lds_loads_done()
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#endif
+}
+
 __device__ __forceinline__ void buf_atomic_add(__amdgpu_buffer_rsrc_t r, int byte_off, float v)
 {
     __builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(v, r, byte_off, 0, 0);

@@ -309,6 +309,23 @@ __global__ __launch_bounds__(256) void k_fdk_filter(const float* __restrict__ in
 // one 8-byte load (4-byte aligned; gfx950 loads need only dword alignment).
 constexpr int ZC = 16;
 
+// Detector column of voxel column (x, y): y' SAD / (U da) + fa0 with 1 / U
+// given, the operations written out so that every mapping rounds alike.
+__device__ __forceinline__ double column_coord(double x, double y, double c, double s, double sda, double iU,
+                                               double fa0)
+{
+    return fma(fma(y, c, -(x * s)) * sda, iU, fa0);
+}
+
+// acc + w0 (row interpolation at the left column) + w1 (at the right one),
+// w0 = w (1 - ta), w1 = w ta: six instructions, the columns' weights shared by
+// the samples of a voxel column (columns first, then rows, then w took seven)
+__device__ __forceinline__ float add_bilinear(float acc, float w0, float w1, float tb, float p00, float p01, float p10,
+                                              float p11)
+{
+    return fmaf(w0, fmaf(tb, p10 - p00, p00), fmaf(w1, fmaf(tb, p11 - p01, p01), acc));
+}
+
 template <bool PAIR>
 __global__ __launch_bounds__(256) void k_fdk_bp(const float* __restrict__ q, const double* __restrict__ trig,
                                                 const float* __restrict__ offsets, int nv, int nx, int ny, int nz,
@@ -327,7 +344,7 @@ __global__ __launch_bounds__(256) void k_fdk_bp(const float* __restrict__ q, con
     const float zc = (float)(z0 + (izc + 0.5) * vz), vzf = (float)vz;   // first voxel's z, step
     const int kn = min(ZC, nz - izc);
     const double ha = na * da * 0.5, hb = nb * db * 0.5;
-    const double inv_da = 1.0 / da;
+    const double inv_da = 1.0 / da, sda = SAD * inv_da, fa0 = ha * inv_da - ai;
     const float inv_db = (float)(1.0 / db);
     const float fb0 = (float)(hb / db - bi);
     const float nb1 = (float)(nb - 1);
@@ -340,14 +357,13 @@ __global__ __launch_bounds__(256) void k_fdk_bp(const float* __restrict__ q, con
         const double U = SID + x * c + y * s;
         if (!(U > 0.0)) continue;
         const double iU = rcp64(U);
-        const double mag = SAD * iU;
-        const double fa = ((-x * s + y * c) * mag + ha) * inv_da - ai;
+        const double fa = column_coord(x, y, c, s, sda, iU, fa0);
         if (!(fa >= 0.0 && fa <= (double)(na - 1))) continue;
         const int ia0 = min((int)floor(fa), max(na - 2, 0));
         const float ta = (float)(fa - ia0);
         const float wr = (float)(SID * iU);
-        const float w = wr * wr;
-        const float mb = (float)mag * inv_db;
+        const float w = wr * wr, w1 = no_contract(w * ta), w0 = w - w1;
+        const float mb = (float)(SAD * iU) * inv_db;
         const int ia1 = min(ia0 + 1, na - 1);
         // branch-free over the ZC voxels, loads first, so all of them are in
         // flight together: a row coordinate outside the detector is clamped for
@@ -366,16 +382,14 @@ __global__ __launch_bounds__(256) void k_fdk_bp(const float* __restrict__ q, con
             for (int k = 0; k < ZC; ++k) {
                 const float fb = fmaf((float)k, dzb, fbs);
                 const int ib0 = (int)fb;
-                tb[k] = fb - (float)ib0;
+                tb[k] = __builtin_amdgcn_fractf(fb);    // fb >= 0: fb - ib0 exactly
                 const unsigned o0 = 4u * (unsigned)(__mul24(ib0, na) + ia0), o1 = o0 + rowstep;
                 __builtin_memcpy(&p0[k], qb + o0, 8);
                 __builtin_memcpy(&p1[k], qb + o1, 8);
             }
 #pragma unroll
             for (int k = 0; k < ZC; ++k) {
-                const float top = fmaf(ta, p0[k].y - p0[k].x, p0[k].x);
-                const float bot = fmaf(ta, p1[k].y - p1[k].x, p1[k].x);
-                acc[k] = fmaf(w, fmaf(tb[k], bot - top, top), acc[k]);
+                acc[k] = add_bilinear(acc[k], w0, w1, tb[k], p0[k].x, p0[k].y, p1[k].x, p1[k].y);
             }
             continue;
         }
@@ -403,9 +417,7 @@ __global__ __launch_bounds__(256) void k_fdk_bp(const float* __restrict__ q, con
         }
 #pragma unroll
         for (int k = 0; k < ZC; ++k) {
-            const float top = fmaf(ta, p0[k].y - p0[k].x, p0[k].x);
-            const float bot = fmaf(ta, p1[k].y - p1[k].x, p1[k].x);
-            const float sum = fmaf(w, fmaf(tb[k], bot - top, top), acc[k]);
+            const float sum = add_bilinear(acc[k], w0, w1, tb[k], p0[k].x, p0[k].y, p1[k].x, p1[k].y);
             acc[k] = valid[k] ? sum : acc[k];
         }
     }
@@ -421,10 +433,10 @@ __global__ __launch_bounds__(256) void k_fdk_bp(const float* __restrict__ q, con
 // copies the block's detector footprint into LDS once (the bounding rectangle
 // of the projected voxel-centre box with one cell of margin) and reads every
 // voxel's four taps from there, instead of gathering 16 bytes per voxel and
-// view through the vector cache.  The footprint of view iv + 1 is loaded into
-// registers before view iv is computed and written to the other LDS buffer
-// after it: one barrier per view.  Per voxel and view the arithmetic is
-// k_fdk_bp's, operation for operation, so all mappings give identical images.
+// view through the vector cache.  The footprint of view iv + 1 is fetched
+// into the other LDS buffer while view iv is computed: one barrier per view.
+// Per voxel and view the arithmetic is k_fdk_bp's, operation for operation,
+// so all mappings give identical images.
 // A view whose footprint exceeds RW x RH cells is gathered from global
 // memory, as k_fdk_bp does.  Footprints are bounded only when every voxel
 // centre lies in front of the source (U > 0 for every view), which the
@@ -438,12 +450,25 @@ __global__ __launch_bounds__(256) void k_fdk_bp(const float* __restrict__ q, con
 // and a third of the HBM traffic, but slower, since one workgroup per CU
 // leaves nothing to run while its waves wait at the per-view barrier).
 //
-// LDS rows have a fixed stride of RW + 4 floats: a voxel's four taps are two
-// ds_read2_b32 at constant offsets (0, 1) and (SRS, SRS + 1) from one
-// address.  Staging: float4 slot j of thread t is float4 t + j T of the
-// footprint (T threads, RW / 4 float4 per row), one 16-byte load whose
-// address is a per-view scalar plus a per-thread constant; the lanes of a
-// wave cover whole rows, or runs of 16 float4 of 4 rows.
+// What bounds the default: vector issue (ten instructions per sample, about
+// 14 with the column's projection: busy 88 % of the time) and, close behind,
+// LDS (two ds_read2_b32 per sample from one address, at constant offsets
+// (0, 1) and (SRS, SRS + 1): busy 77 %).  512 x 512 x 256 voxels, 408 views of
+// 1024 x 768: 14.0 -> 10.8 ms, from
+//   - rows loaded straight into LDS, one dword per lane (13.7 -> 12.5).  Held
+//     in registers under a branch per 16-byte slot, each load first waited for
+//     the one before it, and a view cost three memory latencies;
+//   - the ways a column's samples are read as one branch after another, which
+//     keeps the accumulators in place (nested, the compiler copied all of them
+//     per view), the taps of the next two samples read ahead and their LDS
+//     address formed by one multiply-add (12.5 -> 11.7);
+//   - a row stride of 77 floats instead of 68, odd and far from the bank
+//     count: with 8 x 8 columns to a wave the rows its taps lie on, up to six
+//     apart, fall on other banks (11.7 -> 10.8; 71: 11.1; 72: 15.0).
+// Blocks 32 voxels tall (half the projections, but three workgroups on a CU)
+// gained 0.3 ms here and lost a quarter on 128^3, single-wave blocks of 8 x 8
+// columns without barriers ask for 2.3 times the footprint bytes (17.1), and
+// blocks dealt to the XCDs in contiguous ranges cost 1.7 ms.
 constexpr int SZ = 16;          // voxels per thread along z
 
 struct Foot {
@@ -518,15 +543,6 @@ __device__ int4 fdk_footprints(const double* __restrict__ trig, const float* __r
     return make_int4(ua0, vb0, staged ? ws >> 2 : 0, H);
 }
 
-// 16 bytes from a 4-byte aligned address (gfx950 global loads need only dword
-// alignment), returned by value so the destination stays in registers
-__device__ __forceinline__ float4 load16(const char* p)
-{
-    float4 v;
-    __builtin_memcpy(&v, p, 16);
-    return v;
-}
-
 __device__ __forceinline__ Foot foot_of(const int4& grp, int g)
 {
     Foot f;
@@ -541,7 +557,7 @@ template <int BXS, int BYS, int NWV, int RW, int RH>
 struct StagedShape {
     static constexpr int T = 64 * NWV;                 // threads
     static constexpr int CPT = BXS * BYS / T;          // voxel columns per thread
-    static constexpr int SRS = RW + 4;                 // LDS row stride (floats)
+    static constexpr int SRS = RW + (RW > 64 ? 4 : 13);    // LDS row stride (floats)
     static constexpr int R4 = RW / 4;                  // float4 per footprint row
     static constexpr int SNJ = RH * R4 / T;            // staging slots per thread and view
     static_assert(CPT * T == BXS * BYS && SNJ * T == RH * R4 && RW % 4 == 0, "block shape");
@@ -557,7 +573,10 @@ __global__ __launch_bounds__(64 * NWV, (RW > 64 ? 1 : 16 / NWV)) void k_fdk_bp_s
 {
     using S = StagedShape<BXS, BYS, NWV, RW, RH>;
     constexpr int CPT = S::CPT, SRS = S::SRS, SNJ = S::SNJ, T = S::T, R4 = S::R4;
-    __shared__ float4 lds4[2][RH * SRS / 4];
+    constexpr bool DMA = RW <= 64;      // loads straight into LDS: a row is at most one wave's dwords
+    static_assert(!DMA || 2 * RH * SRS * 4 <= 65536, "their LDS offsets have 16 bits");
+    __shared__ float4 lds4[2][(RH * SRS + 3) / 4];
+    const int lds0 = (int)(size_t)(__attribute__((address_space(3))) const void*)&lds4[0][0];
     const int tid = threadIdx.x;
     // Block coordinates.  XCDMAP: a 1-D grid (a multiple of 8) whose
     // workgroups the hardware deals to the 8 XCDs in turn (id mod 8) is
@@ -586,8 +605,11 @@ __global__ __launch_bounds__(64 * NWV, (RW > 64 ? 1 : 16 / NWV)) void k_fdk_bp_s
     // T is a multiple of BXS, so all of them share x and step y by T / BXS
     static_assert(T % BXS == 0, "columns of a thread share x");
     constexpr int YSTEP = T / BXS;
-    const int ix = bxi * BXS + tid % BXS;
-    const int iy0 = byi * BYS + tid / BXS;
+    // 16 x 16 columns: a wave takes 8 x 8 of them, whose taps lie closer
+    // together than those of 16 x 4 (10.8 instead of 11.6 ms)
+    const bool quad = BXS == 16 && BYS == 16 && NWV == 4;
+    const int ix = bxi * BXS + (quad ? (tid & 7) + 8 * ((tid >> 6) & 1) : tid % BXS);
+    const int iy0 = byi * BYS + (quad ? ((tid >> 3) & 7) + 8 * (tid >> 7) : tid / BXS);
     const double x = x0 + (ix + 0.5) * vx;
     float acc[CPT][SZ];
 #pragma unroll
@@ -600,7 +622,7 @@ __global__ __launch_bounds__(64 * NWV, (RW > 64 ? 1 : 16 / NWV)) void k_fdk_bp_s
     // na/2) - ai (the launcher passes ai + 0.5, bi + 0.5)
     const double ha = PIX ? (double)(na / 2) * da : na * da * 0.5;
     const double hb = PIX ? (double)(nb / 2) * db : nb * db * 0.5;
-    const double inv_da = 1.0 / da, inv_db64 = 1.0 / db;
+    const double inv_da = 1.0 / da, inv_db64 = 1.0 / db, sda = SAD * inv_da, fa0 = ha * inv_da - ai;
     const float inv_db = (float)inv_db64;
     const float fb0 = (float)(hb / db - bi);
     const float nb1 = (float)(nb - 1);
@@ -632,26 +654,39 @@ __global__ __launch_bounds__(64 * NWV, (RW > 64 ? 1 : 16 / NWV)) void k_fdk_bp_s
         return fdk_footprints<PIX, CYL>(trig, angles, offsets, nv, v0, cx0, cx1, cy0, cy1, cz0, cz1, SID, SAD, ha, hb,
                                    inv_da, ai, inv_db64, bi, na, nb, RW, RH);
     };
-    // this thread's staging cells: float4 tid + j T of the footprint, row
+    // !DMA: this thread's staging cells: float4 tid + j T of the footprint, row
     // (tid + j T) / R4, cells 4 m .. 4 m + 3 with m = tid % R4 (T is a
     // multiple of R4, so m is the same for every j)
     const int m4 = 4 * (tid % R4);
     const int rsub = tid / R4;                          // row of slot 0
     constexpr int RSTEP = T / R4;                       // rows between slots (R4 <= T)
     static_assert(R4 <= T, "one footprint row per slot set");
-    const unsigned goff = 4u * (unsigned)(rsub * na + m4);    // bytes, within the view (< 2^31)
+    const unsigned goff = 4u * (unsigned)(rsub * na + m4);    // bytes from the footprint's first cell
     const int soff = rsub * SRS + m4;                         // floats, within an LDS buffer
-    auto stage_load = [&](const Foot& f, int jv, float4 (&st)[SNJ]) {
-        if (f.wq == 0) return;
+    auto stage_load = [&](const Foot& f, int jv, auto& st) {
+        // the footprint as a buffer of its own bytes: rows past it lie past its
+        // end and are not read (an unstaged view: an empty buffer)
+        const size_t first = (size_t)nb * na * min(jv, nv - 1) + (size_t)(f.vb0 * na + f.ua0);
+        const auto fp = make_rsrc(q + first, f.wq == 0 ? 0u : 4u * (unsigned)((f.H - 1) * na + 4 * f.wq));
         const bool col_ok = m4 < 4 * f.wq;
-        const char* qb = reinterpret_cast<const char*>(q + (size_t)nb * na * jv);
 #pragma unroll
         for (int j = 0; j < SNJ; ++j) {
-            const int r0 = RSTEP * j;
-            if (col_ok && r0 + rsub < f.H) st[j] = load16(qb + 4u * (unsigned)((f.vb0 + r0) * na + f.ua0) + goff);
+            const unsigned o = goff + 4u * (unsigned)(RSTEP * j) * (unsigned)na;    // < 2^32: RH rows of na < 2^23
+            st[j] = buf_load4(fp, (int)(col_ok ? o : 0x80000000u));
         }
     };
-    auto stage_store = [&](const Foot& f, int b, const float4 (&st)[SNJ]) {
+    // DMA: a row of up to 64 cells is one load straight into LDS; wave w takes
+    // rows w, w + NWV, ...
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    auto stage_dma = [&](const Foot& f, int jv, int b) {
+        const size_t first = (size_t)nb * na * min(jv, nv - 1) + (size_t)(f.vb0 * na + f.ua0);
+        const rsrc_words fp = make_rsrc_words(q + first, f.wq == 0 ? 0u : 4u * (unsigned)((f.H - 1) * na + 4 * f.wq));
+        const int lane_off = (tid & 63) < 4 * f.wq ? 4 * (tid & 63) : (int)0x80000000u;
+        const unsigned lds = (unsigned)(lds0 + b * (int)sizeof(lds4[0]));
+        const int rows = f.wq == 0 ? 0 : f.H;
+        for (int r = wave; r < rows; r += NWV) buf_load_lds(fp, lane_off, 4u * (unsigned)r * (unsigned)na, lds + 4u * SRS * r);
+    };
+    auto stage_store = [&](const Foot& f, int b, const auto& st) {
         if (f.wq == 0) return;
         const bool col_ok = m4 < 4 * f.wq;
         float* lb = reinterpret_cast<float*>(&lds4[b][0]);
@@ -663,11 +698,18 @@ __global__ __launch_bounds__(64 * NWV, (RW > 64 ? 1 : 16 / NWV)) void k_fdk_bp_s
     };
     int4 grp = footprints(0);
     Foot cur = foot_of(grp, 0);
-    {
+    if constexpr (DMA) {
+        stage_dma(cur, 0, 0);
+        lds_loads_done();
+    } else {
         float4 st[SNJ];
         stage_load(cur, 0, st);
         stage_store(cur, 0, st);
     }
+    // the current view's trig and offset, loaded a view ahead
+    double cth, sth;
+    trig_of(0, cth, sth);
+    float off = offsets ? offsets[0] : 0.0f;
     __syncthreads();
     for (int iv = 0; iv < nv; ++iv) {
         const int jn = iv + 1;
@@ -676,102 +718,140 @@ __global__ __launch_bounds__(64 * NWV, (RW > 64 ? 1 : 16 / NWV)) void k_fdk_bp_s
             if ((jn & 7) == 0) grp = footprints(jn);
             nxt = foot_of(grp, jn & 7);
         }
-        float4 st[SNJ];
-        stage_load(nxt, jn, st);
+        float4 st[DMA ? 1 : SNJ];
+        if constexpr (DMA)
+            stage_dma(nxt, jn, jn & 1);
+        else
+            stage_load(nxt, jn, st);
         // view iv, from LDS buffer iv & 1 (or from global memory)
         const float* qv = q + (size_t)nb * na * iv;
-        const float off = offsets ? offsets[iv] : 0.0f;
-        double cth, sth;
-        trig_of(iv, cth, sth);
         // The next view's cells go to the other buffer (nobody reads it before
         // the barrier below) once the first column is done: with several
         // columns per thread their registers are then free for the others.
 #pragma unroll
         for (int c = 0; c < CPT; ++c) {
-            do {   // one column's SZ samples; break leaves it
+            // one column's SZ samples, by how they are read: 0 none, 1 from LDS,
+            // 2 from LDS with rows past the detector, 3 from global memory
+            // (one after the other, not nested: the accumulators stay in place)
+            int how = 0, ia0 = 0;
+            float ta = 0.0f, w0 = 0.0f, w1 = 0.0f, fbs = 0.0f, dzb = 0.0f;
+            do {
                 const int iy = iy0 + c * YSTEP;
                 const double y = y0 + (iy + 0.5) * vy;
                 const double U = SID + x * cth + y * sth;
                 if (!(ix < nx && iy < ny && U > 0.0)) break;
                 const double iU = rcp64(U);
-                const double mag = SAD * iU;
                 // CYL (cylindrical detector, the voxel-driven op only): the
                 // column from the ray's in-plane angle, atan2 in FP32 as the
                 // op computes it (pixel.cu.cc:70-71)
                 const double fa = CYL ? (double)atan2f((float)(-x * sth + y * cth), (float)U) * inv_da + ha * inv_da - ai
-                                      : ((-x * sth + y * cth) * mag + ha) * inv_da - ai;
+                                      : column_coord(x, y, cth, sth, sda, iU, fa0);
                 // PIX: 0 <= a < na - 1 (the op skips a view whose 2 x 2
                 // neighbourhood leaves the detector, pixel.cu.cc:43-50)
                 if (!(fa >= 0.0 && (PIX ? fa < (double)(na - 1) : fa <= (double)(na - 1)))) break;
-                const int ia0 = min((int)floor(fa), na - 2);
-                const float ta = (float)(fa - ia0);
+                ia0 = min((int)floor(fa), na - 2);
+                ta = (float)(fa - ia0);
                 const float wr = (float)(SID * iU);
                 const float w = PIX ? 1.0f : wr * wr;
-                const float mb = (float)mag * inv_db;
+                w1 = no_contract(w * ta);
+                w0 = w - w1;
+                const float mb = (float)(SAD * iU) * inv_db;
                 const float fbv = fmaf(-off, mb, fb0);   // row coordinate of z = 0
-                const float fbs = fmaf(zc, mb, fbv), dzb = no_contract(vzf * mb);
+                dzb = no_contract(vzf * mb);
+                fbs = fmaf(zc, mb, fbv);
                 if (cur.wq > 0) {
-                    // float index of row ib0's tap ia0: ib0 SRS + base
-                    const float* lb = reinterpret_cast<const float*>(&lds4[iv & 1][0]);
-                    const int base = (ia0 - cur.ua0) - cur.vb0 * SRS;
                     // A column whose SZ row coordinates all lie in [0, nb - 1)
                     // (fma is monotone in k: its ends bound it) needs no clamp,
                     // no validity test and no select: the same sums, bitwise.
                     const float fbl = fmaf((float)(SZ - 1), dzb, fbs);
-                    if (kn == SZ && fminf(fbs, fbl) >= 0.0f && fmaxf(fbs, fbl) < nb1) {
-#pragma unroll
-                        for (int k = 0; k < SZ; ++k) {
-                            const float fb = fmaf((float)k, dzb, fbs);
-                            const int ib0 = (int)fb;                  // 0 <= fb < nb - 1
-                            const float tb = fb - (float)ib0;
-                            const float* p = lb + (__mul24(ib0, SRS) + base);
-                            const float p00 = p[0], p01 = p[1], p10 = p[SRS], p11 = p[SRS + 1];
-                            const float top = fmaf(ta, p01 - p00, p00);
-                            const float bot = fmaf(ta, p11 - p10, p10);
-                            acc[c][k] = fmaf(w, fmaf(tb, bot - top, top), acc[c][k]);
-                        }
-                        break;
-                    }
-#pragma unroll
-                    for (int k = 0; k < SZ; ++k) {
-                        const float fb = fmaf((float)k, dzb, fbs);
-                        const float fbc = __builtin_amdgcn_fmed3f(fb, 0.0f, nb1);
-                        // 0 <= fb <= nb - 1 (PIX: < nb - 1)
-                        const bool valid = k < kn && fb == fbc && (!PIX || fb < nb1);
-                        const int ib0 = min((int)fbc, nb - 2);    // fbc >= 0: truncation is floor
-                        const float tb = fbc - (float)ib0;
-                        const float* p = lb + (__mul24(ib0, SRS) + base);
-                        const float p00 = p[0], p01 = p[1], p10 = p[SRS], p11 = p[SRS + 1];
-                        const float top = fmaf(ta, p01 - p00, p00);
-                        const float bot = fmaf(ta, p11 - p10, p10);
-                        const float sum = fmaf(w, fmaf(tb, bot - top, top), acc[c][k]);
-                        acc[c][k] = valid ? sum : acc[c][k];
-                    }
+                    how = kn == SZ && fminf(fbs, fbl) >= 0.0f && fmaxf(fbs, fbl) < nb1 ? 1 : 2;
                 } else {
-                    const char* qb = reinterpret_cast<const char*>(qv);
-#pragma unroll
-                    for (int k = 0; k < SZ; ++k) {
-                        const float fb = fmaf((float)k, dzb, fbs);
-                        const float fbc = __builtin_amdgcn_fmed3f(fb, 0.0f, nb1);
-                        const bool valid = k < kn && fb == fbc && (!PIX || fb < nb1);
-                        const int ib0 = min((int)fbc, nb - 2);
-                        const float tb = fbc - (float)ib0;
-                        const unsigned o0 = 4u * (unsigned)(__mul24(ib0, na) + ia0), o1 = o0 + rowstep;
-                        float2 p0, p1;
-                        __builtin_memcpy(&p0, qb + o0, 8);
-                        __builtin_memcpy(&p1, qb + o1, 8);
-                        const float top = fmaf(ta, p0.y - p0.x, p0.x);
-                        const float bot = fmaf(ta, p1.y - p1.x, p1.x);
-                        const float sum = fmaf(w, fmaf(tb, bot - top, top), acc[c][k]);
-                        acc[c][k] = valid ? sum : acc[c][k];
-                        // several columns' accumulators leave no registers for
-                        // every sample's taps in flight at once
-                        if (CPT > 1 && k % 4 == 3) __builtin_amdgcn_sched_barrier(0);
-                    }
+                    how = 3;
                 }
             } while (0);
-            if (c == 0) stage_store(nxt, jn & 1, st);
+            // LDS address of row ib0's tap ia0: 4 ib0 SRS + base (one 24-bit
+            // multiply-add)
+            const int base = lds0 + (iv & 1) * (int)sizeof(lds4[0]) + 4 * ((ia0 - cur.ua0) - cur.vb0 * SRS);
+            auto tap = [&](int ib0) {
+                return (__attribute__((address_space(3))) const float*)(size_t)(unsigned)(__mul24(ib0, 4 * SRS) + base);
+            };
+            if (how == 1) {
+                // groups of GS samples, the next group's taps read before a
+                // group is summed (four: 0.3 ms slower at 512 x 512 x 256)
+                constexpr int GS = 2;
+                float tb[2][GS], p[2][GS][4];
+                auto taps = [&](int g) {
+#pragma unroll
+                    for (int i = 0; i < GS; ++i) {
+                        const int k = g * GS + i;
+                        const float fb = fmaf((float)k, dzb, fbs);
+                        const int ib0 = (int)fb;                           // 0 <= fb < nb - 1
+                        tb[g & 1][i] = __builtin_amdgcn_fractf(fb);        // fb - ib0 exactly
+                        const auto t = tap(ib0);
+                        p[g & 1][i][0] = t[0];
+                        p[g & 1][i][1] = t[1];
+                        p[g & 1][i][2] = t[SRS];
+                        p[g & 1][i][3] = t[SRS + 1];
+                    }
+                };
+                taps(0);
+#pragma unroll
+                for (int g = 0; g < SZ / GS; ++g) {
+                    if (g + 1 < SZ / GS) taps(g + 1);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int i = 0; i < GS; ++i) {
+                        float& a = acc[c][g * GS + i];
+                        const float* t = p[g & 1][i];
+                        a = add_bilinear(a, w0, w1, tb[g & 1][i], t[0], t[1], t[2], t[3]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            if (how == 2) {
+#pragma unroll
+                for (int k = 0; k < SZ; ++k) {
+                    const float fb = fmaf((float)k, dzb, fbs);
+                    const float fbc = __builtin_amdgcn_fmed3f(fb, 0.0f, nb1);
+                    // 0 <= fb <= nb - 1 (PIX: < nb - 1)
+                    const bool valid = k < kn && fb == fbc && (!PIX || fb < nb1);
+                    const int ib0 = min((int)fbc, nb - 2);    // fbc >= 0: truncation is floor
+                    const float tb = fbc - (float)ib0;
+                    const auto p = tap(ib0);
+                    const float p00 = p[0], p01 = p[1], p10 = p[SRS], p11 = p[SRS + 1];
+                    const float sum = add_bilinear(acc[c][k], w0, w1, tb, p00, p01, p10, p11);
+                    acc[c][k] = valid ? sum : acc[c][k];
+                }
+            }
+            if (how == 3) {
+                const char* qb = reinterpret_cast<const char*>(qv);
+#pragma unroll
+                for (int k = 0; k < SZ; ++k) {
+                    const float fb = fmaf((float)k, dzb, fbs);
+                    const float fbc = __builtin_amdgcn_fmed3f(fb, 0.0f, nb1);
+                    const bool valid = k < kn && fb == fbc && (!PIX || fb < nb1);
+                    const int ib0 = min((int)fbc, nb - 2);
+                    const float tb = fbc - (float)ib0;
+                    const unsigned o0 = 4u * (unsigned)(__mul24(ib0, na) + ia0), o1 = o0 + rowstep;
+                    float2 p0, p1;
+                    __builtin_memcpy(&p0, qb + o0, 8);
+                    __builtin_memcpy(&p1, qb + o1, 8);
+                    const float sum = add_bilinear(acc[c][k], w0, w1, tb, p0.x, p0.y, p1.x, p1.y);
+                    acc[c][k] = valid ? sum : acc[c][k];
+                    // several columns' accumulators leave no registers for
+                    // every sample's taps in flight at once
+                    if (CPT > 1 && k % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            if constexpr (!DMA) {
+                if (c == 0) stage_store(nxt, jn & 1, st);
+            }
         }
+        if (jn < nv) {
+            trig_of(jn, cth, sth);
+            off = offsets ? offsets[jn] : 0.0f;
+        }
+        if constexpr (DMA) lds_loads_done();
         __syncthreads();
         cur = nxt;
     }
