@@ -82,7 +82,13 @@ __global__ __launch_bounds__(256) void k_tex_deform(const float* __restrict__ im
 // fixed-point inverse of a displacement field (DeformInvertKernel,
 // deform_tex.cu.cc:78-100): d = (x, y, z) from 0; each iteration
 // x = -mx(i + d), then y = -my(i + d), then z = -mz(i + d), every sample using
-// the components already updated
+// the components already updated.  An iteration is a function of (x, y, z)
+// alone, so a state that comes back bit for bit repeats: after one step
+// nothing changes any more, after two the last iteration's parity says which
+// of the pair it ends on.  A smooth field contracts to either in a few steps
+// (the sampled positions have 2^-17 of a voxel at best), and a wave stops with
+// its last lane; the samples' gathers bound the kernel.  256 x 256 x 160, 30
+// iterations, a smooth field of a few voxels: 1.76 -> 0.35 ms.
 __global__ __launch_bounds__(256) void k_tex_invert(const float* __restrict__ mx, const float* __restrict__ my,
                                                     const float* __restrict__ mz, int nx, int ny, int nz, int iters,
                                                     float* __restrict__ ox, float* __restrict__ oy,
@@ -93,10 +99,19 @@ __global__ __launch_bounds__(256) void k_tex_invert(const float* __restrict__ mx
     if (!voxel_of(id, nx, ny, nz, ix, iy, iz)) return;
     float x = 0.0f, y = 0.0f, z = 0.0f;
     const float fx = (float)ix, fy = (float)iy, fz = (float)iz;
+    const auto same = [](float a, float b) { return __float_as_uint(a) == __float_as_uint(b); };
+    float x1 = 0.0f, y1 = 0.0f, z1 = 0.0f, x2 = 0.0f, y2 = 0.0f, z2 = 0.0f;     // one and two iterations back
     for (int it = 0; it < iters; ++it) {
+        x2 = x1, y2 = y1, z2 = z1;
+        x1 = x, y1 = y, z1 = z;
         x = -tex3(mx, nx, ny, nz, x + fx + 0.5f, y + fy + 0.5f, z + fz + 0.5f);
         y = -tex3(my, nx, ny, nz, x + fx + 0.5f, y + fy + 0.5f, z + fz + 0.5f);
         z = -tex3(mz, nx, ny, nz, x + fx + 0.5f, y + fy + 0.5f, z + fz + 0.5f);
+        if (same(x, x1) && same(y, y1) && same(z, z1)) break;
+        if (it > 0 && same(x, x2) && same(y, y2) && same(z, z2)) {
+            if ((iters - 1 - it) & 1) x = x1, y = y1, z = z1;
+            break;
+        }
     }
     ox[id] = x;
     oy[id] = y;
