@@ -111,29 +111,75 @@ __global__ void k_deform(const float* __restrict__ img, const float* __restrict_
 }
 
 // grad_img[c] += g[i] * w_c(p_i)   (transpose of k_deform in the image)
-__global__ void k_deform_adjoint(const float* __restrict__ g, const float* __restrict__ mx,
-                                 const float* __restrict__ my, const float* __restrict__ mz, int nx, int ny, int nz,
-                                 int boundary, float* __restrict__ gimg, uint32_t gbytes)
+//
+// Bound by the atomics.  Where the next lane's sample lies in the next cell
+// along x (same y and z: the rule wherever the field is smooth), this lane's
+// right corners are that lane's left ones: it takes their values over and adds
+// both at once.  A lane goes through ADJ_ROWS voxels along y and likewise
+// carries the two upper corners on to the next row's lower ones, so a voxel
+// costs 2.5 atomics instead of eight (256 x 256 x 160 voxels, a smooth field:
+// 405 us with eight, 288 with four, 227 so).
+constexpr int ADJ_ROWS = 4;
+__global__ __launch_bounds__(256) void k_deform_adjoint(const float* __restrict__ g, const float* __restrict__ mx,
+                                                        const float* __restrict__ my, const float* __restrict__ mz,
+                                                        int nx, int ny, int nz, int boundary,
+                                                        float* __restrict__ gimg, uint32_t gbytes)
 {
     const int ix = blockIdx.x * blockDim.x + threadIdx.x;
-    const int iy = blockIdx.y;
     const int iz = blockIdx.z;
-    if (ix >= nx) return;
-    const size_t id = (size_t)ix + (size_t)nx * ((size_t)iy + (size_t)ny * iz);
-    const float gv = g[id];
-    const float dx = mx[id], dy = my[id], dz = mz[id];
-    if (gv == 0.0f || !finite3(dx, dy, dz)) return;
-    const Corners c = corners_of(ix, iy, iz, dx, dy, dz, nx, ny, nz);
-    if (boundary == 0 && !c.ok) return;
+    const int lane = threadIdx.x & 63;
     const __amdgpu_buffer_rsrc_t rs = make_rsrc(gimg, gbytes);
+    // a value that is not 0 has its corner inside
+    auto add = [&](int x, int y, int z, float v) {
+        if (v != 0.0f) buf_atomic_add(rs, (int)(((size_t)x + (size_t)nx * ((size_t)y + (size_t)ny * z)) * 4), v);
+    };
+    int px = 0, py = 0, pz = 0;             // corner (px, py, pz) and (px, py, pz + 1) hold up[0], up[1]
+    float up[2] = {0.0f, 0.0f};
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-        const int x = c.x0 + (q & 1), y = c.y0 + ((q >> 1) & 1), z = c.z0 + (q >> 2);
-        const float w = ((q & 1) ? c.fx : 1.0f - c.fx) * (((q >> 1) & 1) ? c.fy : 1.0f - c.fy) *
-                        ((q >> 2) ? c.fz : 1.0f - c.fz);
-        if (inside(x, y, z, nx, ny, nz) && w != 0.0f)
-            buf_atomic_add(rs, (int)(((size_t)x + (size_t)nx * ((size_t)y + (size_t)ny * z)) * 4), gv * w);
+    for (int k = 0; k < ADJ_ROWS; ++k) {
+        const int iy = blockIdx.y * ADJ_ROWS + k;
+        const size_t id = (size_t)min(ix, nx - 1) + (size_t)nx * ((size_t)min(iy, ny - 1) + (size_t)ny * iz);
+        const float gv = g[id];
+        const float dx = mx[id], dy = my[id], dz = mz[id];
+        // every lane stays for the exchange; one without a sample has zeros
+        bool live = ix < nx && iy < ny && gv != 0.0f && finite3(dx, dy, dz);
+        Corners c = {};
+        if (live) {
+            c = corners_of(ix, iy, iz, dx, dy, dz, nx, ny, nz);
+            live = boundary != 0 || c.ok;
+        }
+        const int xn = __shfl_down(c.x0, 1), yn = __shfl_down(c.y0, 1), zn = __shfl_down(c.z0, 1);
+        const bool next_live = __shfl_down((int)live, 1) != 0;
+        const bool hand = lane != 63 && live && next_live && xn == c.x0 + 1 && yn == c.y0 && zn == c.z0;
+        float left[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int y = c.y0 + (q & 1), z = c.z0 + (q >> 1);
+            float v[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const float w =
+                    (h ? c.fx : 1.0f - c.fx) * ((q & 1) ? c.fy : 1.0f - c.fy) * ((q >> 1) ? c.fz : 1.0f - c.fz);
+                v[h] = live && w != 0.0f && inside(c.x0 + h, y, z, nx, ny, nz) ? gv * w : 0.0f;
+            }
+            const float given = __shfl_up(hand ? v[1] : 0.0f, 1);
+            left[q] = v[0] + (lane != 0 ? given : 0.0f);
+            if (!hand) add(c.x0 + 1, y, z, v[1]);
+        }
+        if (live && px == c.x0 && py == c.y0 && pz == c.z0) {
+            left[0] += up[0];
+            left[2] += up[1];
+        } else {
+            add(px, py, pz, up[0]);
+            add(px, py, pz + 1, up[1]);
+        }
+        add(c.x0, c.y0, c.z0, left[0]);
+        add(c.x0, c.y0, c.z0 + 1, left[2]);
+        px = c.x0, py = c.y0 + 1, pz = c.z0;
+        up[0] = left[1], up[1] = left[3];
     }
+    add(px, py, pz, up[0]);
+    add(px, py, pz + 1, up[1]);
 }
 
 // d<g, warp(img, m)>/dm at each voxel (the derivative of the trilinear
@@ -234,8 +280,8 @@ int nefct_deform_adjoint(const float* grad_out, const float* mx, const float* my
     size_t blocks = (n + 255) / 256;
     if (blocks > 8192) blocks = 8192;
     hipLaunchKernelGGL(k_fill0, dim3((unsigned)blocks), dim3(256), 0, s, grad_image, n);
-    hipLaunchKernelGGL(k_deform_adjoint, dim3((nx + 255) / 256, ny, nz), dim3(256), 0, s, grad_out, mx, my, mz, nx,
-                       ny, nz, boundary, grad_image, (uint32_t)(n * 4));
+    hipLaunchKernelGGL(k_deform_adjoint, dim3((nx + 255) / 256, (ny + ADJ_ROWS - 1) / ADJ_ROWS, nz), dim3(256), 0, s,
+                       grad_out, mx, my, mz, nx, ny, nz, boundary, grad_image, (uint32_t)(n * 4));
     NEFCT_CHECK_LAUNCH();
     return NEFCT_OK;
 }
