@@ -132,6 +132,20 @@ __device__ __forceinline__ FanRay fan_ray(const VolDev& V, const DetDev& G, cons
     return r;
 }
 
+// Paths within 1/64 of a grid axis cross a face so slowly that the rounding of
+// an FP32 coordinate (4e-6 cells at 64 cells from the middle) moves the
+// crossing by 1e-3 slabs and more.  A ray's own coordinates are rounded about
+// the middle of its own path, which differs from its column's where the ray
+// leaves the volume in z, so on these paths (2 % of them) the rays work out
+// their crossings themselves (FanOwn) and the table holds slabs: f0 = the
+// cell before the crossing, dt = which part of the slab (FAN_WHOLE ...).  A
+// slab whose faces come within FAN_REACH (relative) of a cell face gets both of
+// its parts: a ray may cross there although its column does in the next slab.
+constexpr double FAN_SLOW = 1.0 / 64.0;
+constexpr float FAN_REACH = 0x1p-20f;   // the two coordinates differ by 4 * 2^-24 of the largest at most
+constexpr float FAN_WHOLE = 0.0f, FAN_FIRST = 1.0f, FAN_SECOND = 2.0f, FAN_EMPTY = 3.0f;
+__device__ __forceinline__ bool fan_slow(const FanCol& C) { return fabs(C.ka) < FAN_SLOW && C.ka != 0.0; }
+
 // The one or two in-plane pieces of slab t (transverse cells c0 and, past a
 // crossing, c1), their lengths and the slab's coordinate (from tc).  A piece of
 // no length is dropped.  ha = half the transverse extent.
@@ -169,27 +183,25 @@ __device__ __forceinline__ FanSlab fan_slab(const FanCol& C, int t, int ha)
         const float a0 = fmaf(ka, tr, Ac), a1 = fmaf(ka, tr + 1.0f, Ac);
         s.c0 = cell_floor(a0) + ha;
         s.c1 = cell_floor(a1) + ha;
+        if (fan_slow(C)) {
+            const float reach = FAN_REACH * (fmaxf(fabsf(a0), fabsf(Ac)) + 1.0f);
+            const float face = floorf(fmaxf(a0, a1) + reach);
+            if (face >= fminf(a0, a1) - reach) {
+                s.c0 = (int)face + ha - (ka > 0.0f ? 1 : 0);
+                s.c1 = (int)face + ha - (ka > 0.0f ? 0 : 1);
+            }
+        }
         cross = s.c0 != s.c1;
         s.d0 = cross ? cross_frac(cell_frac(a0), ika, ka > 0.0f ? ika : 0.0f) : 1.0f;
         s.d1 = 1.0f - s.d0;
     }
     s.ts = tr;
     const bool in = t >= C.s0 && t < C.s1();
-    s.v0 = in && s.d0 > 0.0f;
-    s.v1 = in && cross && s.d1 > 0.0f;
+    const bool parts = cross && fan_slow(C);    // both, whatever the column's own lengths
+    s.v0 = in && (parts || s.d0 > 0.0f);
+    s.v1 = in && cross && (parts || s.d1 > 0.0f);
     return s;
 }
-
-// Paths within 1/64 of a grid axis cross a face so slowly that the rounding of
-// an FP32 coordinate (4e-6 cells at 64 cells from the middle) moves the
-// crossing by 1e-3 slabs and more.  A ray's own coordinates are rounded about
-// the middle of its own path, which differs from its column's where the ray
-// leaves the volume in z, so on these paths (2 % of them) the rays work out
-// their crossings themselves (FanOwn) and the table holds slabs: f0 = the
-// cell before the crossing, dt = which part of the slab (FAN_WHOLE ...).
-constexpr double FAN_SLOW = 1.0 / 64.0;
-constexpr float FAN_WHOLE = 0.0f, FAN_FIRST = 1.0f, FAN_SECOND = 2.0f, FAN_EMPTY = 3.0f;
-__device__ __forceinline__ bool fan_slow(const FanCol& C) { return fabs(C.ka) < FAN_SLOW && C.ka != 0.0; }
 
 // A ray's own in-plane coordinate: a(t) = ka (t - tc - shift) + Ac.
 struct FanOwn {
@@ -255,8 +267,11 @@ __device__ __forceinline__ FanSeg fan_seg(const FanSlab& s, bool second, bool sl
 
 __device__ __forceinline__ FanSeg fan_own_seg(const FanSeg& e, const FanOwn& w)
 {
-    const float a0 = fmaf(w.ka, e.ts - w.shift, w.Ac);
-    const float fa = e.dt == FAN_WHOLE ? 1.0f : cross_frac(a0 - e.f0, w.ika, w.pia);
+    // (by the cells of the slab's two faces, as the per-ray walk finds a crossing)
+    const float a0 = fmaf(w.ka, e.ts - w.shift, w.Ac), a1 = fmaf(w.ka, e.ts - w.shift + 1.0f, w.Ac);
+    const float fa = e.dt == FAN_WHOLE || floorf(a1) == e.f0 ? 1.0f
+                     : floorf(a0) != e.f0                    ? 0.0f
+                                                             : cross_frac(a0 - e.f0, w.ika, w.pia);
     FanSeg r;
     r.ts = e.ts;
     r.f0 = e.dt == FAN_SECOND ? fa : 0.0f;
@@ -544,7 +559,7 @@ void launch_fan_fwd(const Launch& L, float* out, int vgl, hipStream_t s)
 // block, 16 rows of each of the four columns at once, and walk their rays.
 // No barrier is needed between views: a table belongs to its wavefront.
 constexpr int FB = 16;
-constexpr int FAN_ENT = 2 * FB;     // table entries per column: at most 2 FB - 1 pieces, and one empty one
+constexpr int FAN_ENT = 2 * FB;     // table entries per column: two per slab at most, and an empty one after an odd count
 
 constexpr int FAN_HALO = 6;
 
@@ -651,7 +666,8 @@ __device__ __forceinline__ void fan_adjoint_block(const Launch& P, const float* 
                 __builtin_amdgcn_wave_barrier();
                 if (q.v0) tab[p++] = fan_seg(q, false, slow, ha, cell0);
                 if (q.v1) tab[p++] = fan_seg(q, true, slow, ha, cell1);
-                if ((q.v0 || q.v1) && p == n)       // an empty piece in the last one's slab makes the count even
+                // an empty piece in the last one's slab makes the count even
+                if ((q.v0 || q.v1) && p == n && n < FAN_ENT)
                     tab[n] = FanSeg{q.ts, 0.0f, slow ? FAN_EMPTY : 0.0f, q.v1 ? cell1 : cell0};
                 __builtin_amdgcn_wave_barrier();
                 ta = tab[0].ts;
