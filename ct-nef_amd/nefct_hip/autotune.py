@@ -10,7 +10,8 @@ work maps onto the chip (include/nefct_hip.h):
   workgroup (a wavefront is the first 64 of them) and the number of
   neighbouring views each XCD walks together (its L2 reuse).
 
-Which is fastest depends on the volume, detector and view count, so the
+(The exact rule on usual cones has kernels whose shapes are fixed: there the
+candidates time alike.)  Which is fastest depends on the volume, detector and view count, so the
 tuner times the candidates on a sample of the views (the forward on a
 contiguous run, since its order exploits neighbouring views; the adjoint on
 an even spread) and keeps the winner per (device, direction, geometry, mode)

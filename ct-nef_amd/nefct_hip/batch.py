@@ -1,8 +1,9 @@
 """Batched Siddon pair over many problems of uneven size.
 
 One launch per direction covers every problem: the forward's workgroups are
-16x16-ray tasks (one view, neighbouring views dealt to the same XCD) and the
-adjoint's 32x32x16 voxel blocks, numbered across all problems, so small
+tasks of 4 detector columns by 64 rows (one view, neighbouring views dealt to
+the same XCD) and the adjoint's blocks of 16x16 voxel columns (16x16 rays and
+32x32x16 voxels with the reference rule or steep cones), numbered across all problems, so small
 problems do not leave the GPU idle and there is one launch instead of one per
 problem (the reference loops
 in Python over views and phases, nefct/functions/project_t.py:153-159,

@@ -219,8 +219,8 @@ int nefct_batch_plan(nefct_problem* problems, int nprob, unsigned flags, size_t*
                      long long* total_tiles, long long* total_blocks);
 
 /* Forward projection of every problem: one trig/launch-record pass, the
- * padded volume copies, then one launch over the 16x16-ray tasks of all
- * problems, dealt to the XCDs in contiguous ranges.  'host_problems' is the
+ * padded volume copies, then one launch over the tasks (4 detector columns x
+ * 64 rows; 16x16 rays with the reference rule or steep rays) of all problems, dealt to the XCDs in contiguous ranges.  'host_problems' is the
  * planned table, 'device_problems' a device copy of it. */
 int nefct_batch_project(const nefct_problem* host_problems, const nefct_problem* device_problems, int nprob,
                         long long total_tiles, unsigned flags, void* workspace, size_t workspace_bytes, void* stream);
