@@ -1522,25 +1522,27 @@ __global__ __launch_bounds__(64 * NW, 4) void k_siddon_adj_tile(Launch P, const 
 
 // Number of view ranges a block's work is split into.  A workgroup fills a
 // CU, so few blocks leave CUs idle (32 blocks at 64^3) or a last round nearly
-// empty; the ranges' integer sums are added in the workspace (8 B per voxel
-// and range through the L2) and need at least `least` views each to be worth
-// it (8 on fan planes; 2 of the per-ray walk's, ~20 us per view and block).
-// The smallest split whose last round leaves 10 % fewer CUs idle: 64^3 voxels,
-// 128^2 cells, 120 views 2226 -> 135 us (1854 us of it the whole adjoint on
-// 16 CUs, 188 us the maximum's atomics).
-inline int tile_splits(const Launch& L, int tx, int ty, int tz, int least)
+// empty; the ranges' integer sums are added in the workspace, one more launch
+// and about 5 ps per voxel and range (2.6 M voxels in five ranges: 64 us).  The
+// number with the least of both, view_us being a block's time per view (about
+// 6 us on fan planes; 20 to 60 us of the per-ray walk, whose blocks differ
+// more, so the upper end).  With at least eight (fan planes) or two views to a
+// range instead: 64x64x40, 12 / 100 views of 83x52 cells 82 -> 41 / 77 -> 65 us,
+// 32x32x24, 40 views 134 -> 34 us; per ray 53x53x25, 14 views 240 -> 126 us,
+// 192x192x200, 100 views 5169 -> 4657 us (but 85x85x91, 21 views 285 -> 371).
+inline int tile_splits(const Launch& L, int tx, int ty, int tz, double view_us)
 {
     constexpr int CUS = 256;
     const long long blocks = (long long)((L.V.n[0] + tx - 1) / tx) * ((L.V.n[1] + ty - 1) / ty) *
                              ((L.V.n[2] + tz - 1) / tz);
-    const int nv = L.nv;
+    const double voxels = (double)L.V.n[0] * L.V.n[1] * L.V.n[2];
     int best = 1;
-    double eff = 0.0;
-    for (int ns = 1; ns <= 64 && (ns == 1 || nv / ns >= least); ++ns) {
-        const long long w = blocks * ns, rounds = (w + CUS - 1) / CUS;
-        const double e = (double)w / (double)(rounds * CUS);
-        if (e > eff + 0.1) {
-            eff = e;
+    double least = 0.0;
+    for (int ns = 1; ns <= 64 && ns <= L.nv; ++ns) {
+        const double walk = (double)((blocks * ns + CUS - 1) / CUS) * ((L.nv + ns - 1) / ns) * view_us;
+        const double us = walk + (ns > 1 ? 8.0 + 5e-6 * voxels * ns : 0.0);
+        if (ns == 1 || us < 0.97 * least) {
+            least = us;
             best = ns;
         }
     }
@@ -1582,7 +1584,7 @@ template <int TX, int TY, int TZ, int NW, int CS>
 void launch_tile(bool ref, bool fix, const Launch& L, const float* pv, float* image, unsigned long long* sums,
                  const unsigned* maxbits, float sbound, hipStream_t s)
 {
-    const int ns = (fix && NW == 16 && sums) ? tile_splits(L, TX, TY, TZ, 2) : 1;
+    const int ns = (fix && NW == 16 && sums) ? tile_splits(L, TX, TY, TZ, 60.0) : 1;
     if (ns == 1) sums = nullptr;
     const dim3 g((L.V.n[0] + TX - 1) / TX, (L.V.n[1] + TY - 1) / TY, (L.V.n[2] + TZ - 1) / TZ * ns);
     const dim3 b(64 * NW);
@@ -1945,10 +1947,10 @@ void launch_adjoint_tiles(Launch& L, const float* pv, float* image, unsigned* ma
         int nsplit = 1;
         if (sums)
             nsplit = L.fan ? tile_splits(L, FB, FB, (L.V.n[2] + fan_zblocks(L.V.n[2], FAN_TZ) - 1) /
-                                                        fan_zblocks(L.V.n[2], FAN_TZ), 8)
-                     : shape == NEFCT_F_TILE_64x32x8 ? tile_splits(L, 64, 32, 8, 2)
-                     : shape == NEFCT_F_TILE_64x16x16 ? tile_splits(L, 64, 16, 16, 2)
-                     : shape == NEFCT_F_TILE_32x32x16 ? tile_splits(L, 32, 32, 16, 2) : 1;
+                                                        fan_zblocks(L.V.n[2], FAN_TZ), 6.0)
+                     : shape == NEFCT_F_TILE_64x32x8 ? tile_splits(L, 64, 32, 8, 60.0)
+                     : shape == NEFCT_F_TILE_64x16x16 ? tile_splits(L, 64, 16, 16, 60.0)
+                     : shape == NEFCT_F_TILE_32x32x16 ? tile_splits(L, 32, 32, 16, 60.0) : 1;
         if (nsplit == 1) sums = nullptr;
         if (L.fan) {
             const size_t used = sums ? vol : 0;
