@@ -265,7 +265,8 @@ __device__ __forceinline__ FanSeg fan_seg(const FanSlab& s, bool second, bool sl
     return FanSeg{s.ts, second ? s.d0 : 0.0f, second ? s.d1 : s.d0, off};
 }
 
-__device__ __forceinline__ FanSeg fan_own_seg(const FanSeg& e, const FanOwn& w)
+// (slow: this lane's column; the entry of another column is a piece already)
+__device__ __forceinline__ FanSeg fan_own_seg(const FanSeg& e, const FanOwn& w, bool slow)
 {
     // (by the cells of the slab's two faces, as the per-ray walk finds a crossing)
     const float a0 = fmaf(w.ka, e.ts - w.shift, w.Ac), a1 = fmaf(w.ka, e.ts - w.shift + 1.0f, w.Ac);
@@ -274,8 +275,8 @@ __device__ __forceinline__ FanSeg fan_own_seg(const FanSeg& e, const FanOwn& w)
                                                              : cross_frac(a0 - e.f0, w.ika, w.pia);
     FanSeg r;
     r.ts = e.ts;
-    r.f0 = e.dt == FAN_SECOND ? fa : 0.0f;
-    r.dt = e.dt == FAN_EMPTY ? 0.0f : e.dt == FAN_SECOND ? 1.0f - fa : fa;
+    r.f0 = !slow ? e.f0 : e.dt == FAN_SECOND ? fa : 0.0f;
+    r.dt = !slow ? e.dt : e.dt == FAN_EMPTY ? 0.0f : e.dt == FAN_SECOND ? 1.0f - fa : fa;
     r.off = e.off;
     return r;
 }
@@ -368,7 +369,7 @@ __device__ __forceinline__ float fan_forward_pieces(const FanSeg* __restrict__ t
 #pragma unroll
         for (int u = 0; u < FAN_U; ++u) {
             FanSeg s = tab[j + u];
-            if (SLOW) s = fan_own_seg(s, own);
+            if (SLOW) s = fan_own_seg(s, own, true);
             float z = fmaf(kz, s.ts, Zc);
             if (CLAMP) z = __builtin_amdgcn_fmed3f(z, zlo, zhi);
             // (falling: from the cell below, the first of the two in memory)
@@ -511,9 +512,11 @@ __device__ __forceinline__ void fan_forward_wave(const Launch& P, int ia, int ib
     if (ib < G.nb) out[(size_t)ia + (size_t)G.na * ((size_t)ib + (size_t)G.nb * (size_t)iv)] = acc * q.scale;
 }
 
-// Task order as k_siddon's, with tiles of FAN_FW columns x 64 rows.
-__global__ __launch_bounds__(64 * FAN_FW) void k_fan_fwd(Launch P, float* __restrict__ out, int tiles_a, int tiles_b,
-                                                        int v0, int nvc, int vg_log2)
+// Task order as k_siddon's, with tiles of FAN_FW columns x 64 rows.  Held to
+// eight wavefronts per SIMD (64 registers; with 68 the 512 x 512 x 256 forward
+// takes 4 % longer).
+__global__ __launch_bounds__(64 * FAN_FW, 8) void k_fan_fwd(Launch P, float* __restrict__ out, int tiles_a, int tiles_b,
+                                                           int v0, int nvc, int vg_log2)
 {
     __shared__ FanSeg tabs[FAN_FW][FAN_TAB];
     const unsigned per_xcd = gridDim.x >> 3;
@@ -643,7 +646,9 @@ __device__ __forceinline__ void fan_adjoint_block(const Launch& P, const float* 
             const int ia = ia0 + 4 * g + col;
             const FanCol C = fan_col(P, iv, min(ia, G.na - 1));
             const int ha = (C.m() == 0 ? ny : nx) >> 1;
-            const bool slow = __any(fan_slow(C));
+            // the group walks as its slow columns need; every column keeps its
+            // own rule, whichever neighbours a block deals it with
+            const bool slow = fan_slow(C), any_slow = __any(slow);
             int n;
             float ta, tb;       // slab coordinates of the path's ends inside the block
             {
@@ -724,7 +729,7 @@ __device__ __forceinline__ void fan_adjoint_block(const Launch& P, const float* 
 #pragma unroll
                             for (int r = 0; r < R; ++r) {
                                 FanSeg e = entry;
-                                if constexpr (SLOW) e = fan_own_seg(entry, own[r]);
+                                if constexpr (SLOW) e = fan_own_seg(entry, own[r], slow);
                                 const float z = fmaf(kz[r], e.ts, Zc[r]);
                                 const int cz = cell_floor(z);
                                 const int o = e.off + cz * ES;
@@ -773,7 +778,7 @@ __device__ __forceinline__ void fan_adjoint_block(const Launch& P, const float* 
                 using R1 = std::integral_constant<int, 1>;
                 using R2 = std::integral_constant<int, 2>;
                 using R4 = std::integral_constant<int, 4>;
-                if (slow) {
+                if (any_slow) {
                     for (; f0 < nf; f0 += 16) rays(f0, R1{}, std::true_type{});
                 } else {
                     for (; nf - f0 > 48; f0 += 64) rays(f0, R4{}, std::false_type{});
