@@ -739,11 +739,18 @@ __device__ __forceinline__ void fan_adjoint_block(const Launch& P, const float* 
                                 // would put many lanes on one word)
                                 const bool ok = !TEST || (unsigned)(cz - ilo - (down ? 1 : 0)) <= span;
                                 if constexpr (FIX) {
-                                    const float whole = e.dt * sv[r];
+                                    // units of the whole piece to the nearest, the
+                                    // first cell's cut, the rest to the next cell:
+                                    // a piece keeps its length (cut apart, the two
+                                    // lost up to a unit each, and with one value 1e5
+                                    // times the others the image was 1.6e-4 too small)
+                                    const float half = NONNEG ? 0.5f : copysignf(0.5f, sv[r]);
+                                    const float whole = fmaf(e.dt, sv[r], half);
                                     const float raw = fmaf(-e.f0, sv[r], fan_z_frac<SIGN>(z, kz[r], ik[r]));
-                                    const float part = __builtin_amdgcn_fmed3f(raw, 0.0f, whole);
-                                    if (ok) deposit(o, (int)part);
-                                    if (ok && part != whole) deposit(o + next, (int)(whole - part));
+                                    const float part = __builtin_amdgcn_fmed3f(raw, half, whole);
+                                    const int q = (int)part;
+                                    if (ok) deposit(o, q);
+                                    if (ok && part != whole) deposit(o + next, (int)whole - q);
                                 } else {
                                     const float raw = fan_z_frac<SIGN>(z, kz[r], ik[r]) - e.f0;
                                     const float l = __builtin_amdgcn_fmed3f(raw, 0.0f, e.dt), h = e.dt - l;
