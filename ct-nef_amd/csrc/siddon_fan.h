@@ -32,18 +32,20 @@ constexpr int FAN_ZPAD = 2;     // zero border of the z-fastest copy's rows
 // in-plane step in voxels), slabs [s0, s1) inside the box (none when it
 // misses), the transverse coordinate a(t) = Aa + ka t at slab face t; and what
 // its rays have in common: kz = b dk cells per slab and, above the view's
-// z0, Zc = b dz cells at the middle slab tc for detector height b (mm).  (From
-// b itself, which is exactly 0 in a middle row: its ray stays in the source's
+// z0, Zc = b dz cells at the end tz towards the source for detector height b
+// (mm).  (From b itself, which is exactly 0 in a middle row: its ray stays in the source's
 // plane.)  One record per column and view is worked out once per call where
 // the workspace has room: the adjoint reads it in every block it passes.
 struct __align__(16) FanCol {
     double ka, ika, Aa, dk, dz;
     double l2;       // squared in-plane source-detector distance in x voxels (1/L^2 scale)
-    float p2;        // squared in-plane mm per slab
-    int tc, s0;
-    int s1m;         // s1, and the walk axis in bit 30
-    __device__ int s1() const { return s1m & 0x3fffffff; }
-    __device__ int m() const { return s1m >> 30; }
+    double p2;       // squared in-plane mm per slab
+    unsigned slabs;  // s0, s1 (15 bits each: grid sides are at most 16384), walk axis (bit 30), path against it (31)
+    __device__ int s0() const { return slabs & 0x7fff; }
+    __device__ int s1() const { return (slabs >> 15) & 0x7fff; }
+    __device__ int m() const { return (slabs >> 30) & 1; }
+    __device__ int tc() const { return (s0() + s1()) >> 1; }        // middle slab
+    __device__ int tz() const { return slabs >> 31 ? s1() : s0(); } // the end towards the source
 };
 static_assert(sizeof(FanCol) == 64, "read as four 16-byte words");
 
@@ -87,14 +89,12 @@ __device__ __forceinline__ FanCol fan_column(const VolDev& V, const DetDev& G, d
     clip_axis(C.ka, C.ika, C.Aa, 0.0, (double)nt, tin, tout);
     const bool hit = dm != 0.0 && tout > tin;
     const int s0 = max((int)floor(tin), 0), s1 = min((int)ceil(tout), nm);
-    C.s0 = hit ? s0 : 0;
-    const int e = hit && s1 > s0 ? s1 : C.s0;
-    C.s1m = e | (x ? 0 : 1 << 30);
-    C.tc = (C.s0 + e) >> 1;
+    const int b = hit ? s0 : 0, e = hit && s1 > s0 ? s1 : b;
+    C.slabs = (unsigned)b | (unsigned)e << 15 | (x ? 0u : 1u << 30) | (dm < 0.0 ? 1u << 31 : 0u);
     C.dk = V.inv_vs[2] * idm;
-    C.dz = C.dk * ((double)C.tc - um);
+    C.dz = C.dk * ((double)C.tz() - um);
     const double kt = C.ka * vt;
-    C.p2 = (float)fma(kt, kt, vm * vm);
+    C.p2 = fma(kt, kt, vm * vm);
     const double x0 = e0 * V.inv_vs[0], x1 = e1 * V.inv_vs[0];
     C.l2 = fma(x1, x1, x0 * x0);
     return C;
@@ -107,9 +107,18 @@ __device__ __forceinline__ double fan_z0(const VolDev& V, double lift)
     return (lift - V.lo[2]) * V.inv_vs[2] - (double)(V.n[2] >> 1);
 }
 
-// z of a ray over its column's path: z(t) = kz (t - tc) + Zc, in cells from
+// z of a ray over its column's path: z(t) = kz (t - tz) + Zc, in cells from
 // the volume's middle cell (nz / 2); ink = 1 / |kz| (capped: a level ray
 // never reaches the next cell); scale = mm per slab.
+// The origin tz is the path's end towards the source.  A ray that meets the
+// volume at all is between the source's height and its own there, so |Zc| stays
+// within the volume (for a source inside its height) and z carries the rounding
+// of numbers of the volume's size, as in the per-ray walk's coordinate about
+// the ray's own middle.  About the path's middle, where a steep ray is far
+// outside, it was up to 3.5 times that (256 x 256 x 16 voxels, source 62 voxels
+// from the volume's face, slopes above 0.2: 1.4e-6 cells rms, now and in the
+// per-ray walk 4.0e-7).  Slope, reciprocal and length per slab are rounded
+// once, from FP64.
 struct FanRay {
     float kz, Zc, ink, scale;
 };
@@ -120,11 +129,13 @@ __device__ __forceinline__ FanRay fan_ray(const VolDev& V, const DetDev& G, cons
 #pragma clang fp contract(off)
     FanRay r;
     const double b = fma(G.bi + ib, G.db, -(G.nb * G.db * 0.5));
-    r.kz = (float)(b * C.dk);
+    const double kz = b * C.dk, kv = kz * V.vs[2];
+    r.kz = (float)kz;
     r.Zc = (float)fma(b, C.dz, z0);
-    r.ink = fminf(__builtin_amdgcn_rcpf(fabsf(r.kz)), 0x1p40f);
-    const float kv = r.kz * (float)V.vs[2];
-    r.scale = __builtin_amdgcn_sqrtf(fmaf(kv, kv, C.p2));
+    // the hardware reciprocal of the FP32 slope and one step towards 1 / |kz|
+    const float rough = fminf(__builtin_amdgcn_rcpf(fabsf(r.kz)), 0x1p40f);
+    r.ink = fmaf(rough, (float)fma(-fabs(kz), (double)rough, 1.0), rough);
+    r.scale = __builtin_amdgcn_sqrtf((float)fma(kv, kv, C.p2));
     if (flags & NEFCT_F_INV_L2) {
         const double zd = b * V.inv_vs[0];
         r.scale = (float)((double)r.scale / fma(zd, zd, C.l2));
@@ -147,7 +158,7 @@ constexpr float FAN_WHOLE = 0.0f, FAN_FIRST = 1.0f, FAN_SECOND = 2.0f, FAN_EMPTY
 __device__ __forceinline__ bool fan_slow(const FanCol& C) { return fabs(C.ka) < FAN_SLOW && C.ka != 0.0; }
 
 // The one or two in-plane pieces of slab t (transverse cells c0 and, past a
-// crossing, c1), their lengths and the slab's coordinate (from tc).  A piece of
+// crossing, c1), their lengths and the slab's coordinate (from tz).  A piece of
 // no length is dropped.  ha = half the transverse extent.
 // The arithmetic is the per-ray walk's (slab_exact: FP32 coordinates from the
 // middle of the volume and of the path), so the two walks agree to the last
@@ -166,7 +177,7 @@ __device__ __forceinline__ FanSlab fan_slab(const FanCol& C, int t, int ha)
 {
 #pragma clang fp contract(off)
     FanSlab s;
-    const float tr = (float)(t - C.tc);
+    const float tr = (float)(t - C.tc());
     bool cross;
     if (fabs(C.ka) > (double)K_NEAR_ONE) {
         const double a0 = fma(C.ka, (double)t, C.Aa), a1 = fma(C.ka, (double)(t + 1), C.Aa);
@@ -179,7 +190,7 @@ __device__ __forceinline__ FanSlab fan_slab(const FanCol& C, int t, int ha)
         s.d0 = (float)fa;
         s.d1 = (float)(1.0 - fa);
     } else {
-        const float ka = (float)C.ka, ika = (float)C.ika, Ac = (float)(fma(C.ka, (double)C.tc, C.Aa) - ha);
+        const float ka = (float)C.ka, ika = (float)C.ika, Ac = (float)(fma(C.ka, (double)C.tc(), C.Aa) - ha);
         const float a0 = fmaf(ka, tr, Ac), a1 = fmaf(ka, tr + 1.0f, Ac);
         s.c0 = cell_floor(a0) + ha;
         s.c1 = cell_floor(a1) + ha;
@@ -195,15 +206,15 @@ __device__ __forceinline__ FanSlab fan_slab(const FanCol& C, int t, int ha)
         s.d0 = cross ? cross_frac(cell_frac(a0), ika, ka > 0.0f ? ika : 0.0f) : 1.0f;
         s.d1 = 1.0f - s.d0;
     }
-    s.ts = tr;
-    const bool in = t >= C.s0 && t < C.s1();
+    s.ts = (float)(t - C.tz());
+    const bool in = t >= C.s0() && t < C.s1();
     const bool parts = cross && fan_slow(C);    // both, whatever the column's own lengths
     s.v0 = in && (parts || s.d0 > 0.0f);
     s.v1 = in && cross && (parts || s.d1 > 0.0f);
     return s;
 }
 
-// A ray's own in-plane coordinate: a(t) = ka (t - tc - shift) + Ac.
+// A ray's own in-plane coordinate: a(t) = ka (t - tz - shift) + Ac.
 struct FanOwn {
     float ka, ika, pia, Ac, shift;
 };
@@ -214,12 +225,12 @@ __device__ __forceinline__ FanOwn fan_own(const VolDev& V, const DetDev& G, cons
     FanOwn w;
     const double b = fma(G.bi + ib, G.db, -(G.nb * G.db * 0.5));
     const double kz = b * C.dk, uz = z0 + (double)(V.n[2] >> 1);
-    const double A = fma(b, fma(-C.dk, (double)C.tc, C.dz), uz);      // z at slab face 0
+    const double A = fma(b, fma(-C.dk, (double)C.tz(), C.dz), uz);      // z at slab face 0
     double tin = 0.0, tout = 16384.0;
     clip_axis(kz, kz != 0.0 ? rcp64(kz) : 0.0, A, 0.0, (double)V.n[2], tin, tout);
-    const int s0 = max(C.s0, (int)floor(fmin(tin, 16384.0))), s1 = min(C.s1(), (int)ceil(fmax(tout, 0.0)));
+    const int s0 = max(C.s0(), (int)floor(fmin(tin, 16384.0))), s1 = min(C.s1(), (int)ceil(fmax(tout, 0.0)));
     const int tc = (s0 + s1) >> 1;
-    w.shift = (float)(tc - C.tc);
+    w.shift = (float)(tc - C.tz());
     w.Ac = (float)(fma(C.ka, (double)tc, C.Aa) - ha);
     w.ka = (float)C.ka;
     w.ika = (float)C.ika;
@@ -413,13 +424,13 @@ __device__ __forceinline__ void fan_forward_wave(const Launch& P, int ia, int ib
     FanOwn own = {};
     if (slow) own = fan_own(V, G, C, vz0, min(ib, G.nb - 1), ha);
     float kz = q.kz, Zc = q.Zc, ink = q.ink;
-    float lo = 3.0e38f, hi = -3.0e38f;      // slabs (from tc) that some ray spends inside the volume
+    float lo = 3.0e38f, hi = -3.0e38f;      // slabs (from tz) that some ray spends inside the volume
     bool rests = false;
-    const float e0 = (float)(C.s0 - C.tc), e1 = (float)(C.s1() - C.tc);
+    const float e0 = (float)(C.s0() - C.tz()), e1 = (float)(C.s1() - C.tz());
     const float zlo = (float)(-hz) - 0.0625f, zhi = (float)(nz - hz) + 0.0625f;
     {
         const float za = fmaf(kz, e0, Zc), zb = fmaf(kz, e1, Zc);
-        if (C.s1() > C.s0 && ib < G.nb && fmaxf(za, zb) > zlo && fminf(za, zb) < zhi) {
+        if (C.s1() > C.s0() && ib < G.nb && fmaxf(za, zb) > zlo && fminf(za, zb) < zhi) {
             // slab coordinates where z passes the (widened) faces; |kz| < 2^-20 stays inside or outside
             lo = e0;
             hi = e1;
@@ -445,9 +456,9 @@ __device__ __forceinline__ void fan_forward_wave(const Launch& P, int ia, int ib
     hi = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, hi)));
     float acc = 0.0f;
     if (lo < hi) {
-        const int t0 = __builtin_amdgcn_readfirstlane(max(C.s0, C.tc + (int)floorf(lo)));
-        const int t1 = __builtin_amdgcn_readfirstlane(min(C.s1(), C.tc + (int)ceilf(hi)));
-        const float w0 = (float)(t0 - C.tc), w1 = (float)(t1 - C.tc);
+        const int t0 = __builtin_amdgcn_readfirstlane(max(C.s0(), C.tz() + (int)floorf(lo)));
+        const int t1 = __builtin_amdgcn_readfirstlane(min(C.s1(), C.tz() + (int)ceilf(hi)));
+        const float w0 = (float)(t0 - C.tz()), w1 = (float)(t1 - C.tz());
         const float za = fmaf(kz, w0, Zc), zb = fmaf(kz, w1, Zc);
         // no ray's two cells leave -2 .. nz + 1 over [t0, t1]: no clamp
         const float down = kz < 0.0f ? 1.0f : 0.0f;
