@@ -34,6 +34,12 @@ __device__ __forceinline__ float4 buf_load4(__amdgpu_buffer_rsrc_t r, int byte_o
 // as assembly because the compiler holds back every later LDS read until such
 // loads have landed: the caller waits with lds_loads_done() before the barrier
 // that hands the cells over.
+// A buffer load may read a scalar register five wait states after a vector
+// instruction (readfirstlane) wrote it at the earliest, and inside assembly
+// nothing keeps that distance: the buffer's words are waited for once, where
+// they are made, and the offset goes through a scalar move, which also is the
+// wait state between m0 and the load (1 % of the FDK backprojection of
+// 512 x 512 x 256 voxels; a five-state wait in every load: 2 %).
 typedef int rsrc_words __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ rsrc_words make_rsrc_words(const void* p, uint32_t nbytes)
 {
@@ -43,17 +49,21 @@ __device__ __forceinline__ rsrc_words make_rsrc_words(const void* p, uint32_t nb
     r.y = __builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32) & 0xffff);
     r.z = __builtin_amdgcn_readfirstlane((int)nbytes);
     r.w = 0x00020000;
+#ifdef __HIP_DEVICE_COMPILE__
+    asm volatile("s_nop 4" : : "s"(r));
+#endif
     return r;
 }
 
 __device__ __forceinline__ void buf_load_lds(rsrc_words r, int lane_off, unsigned off, unsigned lds)
 {
 #ifdef __HIP_DEVICE_COMPILE__
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
-                 :
+    int at;
+    asm volatile("s_mov_b32 m0, %1\n\ts_mov_b32 %0, %4\n\tbuffer_load_dword %2, %3, %0 offen lds"
+                 : "=&s"(at)
                  : "s"(__builtin_amdgcn_readfirstlane((int)lds)), "v"(lane_off), "s"(r),
                    "s"(__builtin_amdgcn_readfirstlane((int)off))
-                 : "memory");
+                 : "memory", "m0");
 #endif
 }
 

@@ -574,6 +574,7 @@ __global__ __launch_bounds__(64 * NWV, (RW > 64 ? 1 : 16 / NWV)) void k_fdk_bp_s
     using S = StagedShape<BXS, BYS, NWV, RW, RH>;
     constexpr int CPT = S::CPT, SRS = S::SRS, SNJ = S::SNJ, T = S::T, R4 = S::R4;
     constexpr bool DMA = RW <= 64;      // loads straight into LDS: a row is at most one wave's dwords
+    static_assert(!DMA || SRS >= 64, "a load writes 64 cells of a row, whatever the footprint's width");
     static_assert(!DMA || 2 * RH * SRS * 4 <= 65536, "their LDS offsets have 16 bits");
     __shared__ float4 lds4[2][(RH * SRS + 3) / 4];
     const int lds0 = (int)(size_t)(__attribute__((address_space(3))) const void*)&lds4[0][0];
