@@ -1793,27 +1793,48 @@ int validate(const int grid[3], const float center[3], const float size[3], cons
     return NEFCT_OK;
 }
 
+// A call's geometry as the kernels take it.
+__host__ __device__ inline void geometry_of(const int grid[3], const float center[3], const float size[3], float SID,
+                                            float SAD, int na, float da, float ai, int nb, float db, float bi, int cyl,
+                                            VolDev& V, DetDev& G)
+{
+    for (int i = 0; i < 3; ++i) {
+        V.n[i] = grid[i];
+        V.vs[i] = (double)size[i] / grid[i];
+        V.inv_vs[i] = 1.0 / V.vs[i];
+        V.lo[i] = (double)center[i] - (double)size[i] * 0.5;
+    }
+    G.cyl = cyl;
+    G.sid = SID;
+    G.sad = SAD;
+    G.na = na;
+    G.nb = nb;
+    G.da = da;
+    G.ai = ai;
+    G.db = db;
+    G.bi = bi;
+}
+
+// Whether a call's rays are walked on fan planes (siddon_fan.h) or each by its
+// own lane.  Of the adjoint's variants the slab windows and the float sums in a
+// fixed order keep the per-ray kernels: on fan planes they would be the float
+// atomics' blocks, 64^3 voxels, 60 views of 128^2 cells in 3305 us against 538
+// (windows), and the same blocks with one wavefront each, 5239 against 1788 us.
+bool walks_fan_planes(const VolDev& V, const DetDev& G, unsigned flags, bool adjoint)
+{
+    if (!fan_ok(V, G, flags)) return false;
+    const unsigned ordered = NEFCT_F_ADJ_FLOAT_ATOMIC | NEFCT_F_DETERMINISTIC;
+    if (adjoint && ((flags & NEFCT_F_ADJ_WINDOW) || (flags & ordered) == ordered)) return false;
+    return true;
+}
+
 Launch make_launch(const int grid[3], const float center[3], const float size[3], int nv, float SID, float SAD,
                    int na, float da, float ai, int nb, float db, float bi, int cyl, unsigned flags, char* ws,
-                   const WsPlan& p, const float* zoff = nullptr)
+                   const WsPlan& p, bool adjoint, const float* zoff = nullptr)
 {
     Launch L;
     L.zoff = zoff;
-    for (int i = 0; i < 3; ++i) {
-        L.V.n[i] = grid[i];
-        L.V.vs[i] = (double)size[i] / grid[i];
-        L.V.inv_vs[i] = 1.0 / L.V.vs[i];
-        L.V.lo[i] = (double)center[i] - (double)size[i] * 0.5;
-    }
-    L.G.cyl = cyl;
-    L.G.sid = SID;
-    L.G.sad = SAD;
-    L.G.na = na;
-    L.G.nb = nb;
-    L.G.da = da;
-    L.G.ai = ai;
-    L.G.db = db;
-    L.G.bi = bi;
+    geometry_of(grid, center, size, SID, SAD, na, da, ai, nb, db, bi, cyl, L.V, L.G);
     L.Ly.xf = (float*)(ws + p.xf_off);
     L.Ly.yf = (float*)(ws + p.yf_off);
     L.Ly.xf_bytes = (uint32_t)(p.xf_elems * 4);
@@ -1825,7 +1846,7 @@ Launch make_launch(const int grid[3], const float center[3], const float size[3]
     L.nv = nv;
     L.flags = flags;
     L.sbound = scale_bound(L.V, L.G, flags);
-    L.fan = fan_ok(L.V, L.G, flags) ? 1 : 0;
+    L.fan = walks_fan_planes(L.V, L.G, flags, adjoint) ? 1 : 0;
     L.cols = nullptr;
     return L;
 }
@@ -1865,7 +1886,7 @@ int run_forward(const float* image, const int grid[3], const float center[3], co
     if (!workspace || wsbytes < p.total) return NEFCT_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
     char* ws = (char*)workspace;
-    Launch L = make_launch(grid, center, size, nv, SID, SAD, na, da, ai, nb, db, bi, cyl, flags, ws, p, zoff);
+    Launch L = make_launch(grid, center, size, nv, SID, SAD, na, da, ai, nb, db, bi, cyl, flags, ws, p, false, zoff);
     if (L.fan) {
         // the z-fastest copy fits the space of the two padded copies
         launch_fan_prep(image, grid, L.Ly.xf, angles, nv, (double*)(ws + p.trig_off), s);
@@ -1900,14 +1921,13 @@ int run_adjoint(const float* pv, const int grid[3], const float center[3], const
     if (!workspace || wsbytes < p.total) return NEFCT_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
     char* ws = (char*)workspace;
-    Launch L = make_launch(grid, center, size, nv, SID, SAD, na, da, ai, nb, db, bi, cyl, flags, ws, p, zoff);
+    Launch L = make_launch(grid, center, size, nv, SID, SAD, na, da, ai, nb, db, bi, cyl, flags, ws, p, true, zoff);
     const int nx = grid[0], ny = grid[1], nz = grid[2];
     const bool ref = (flags & NEFCT_F_REF_SLAB) != 0;
     unsigned* maxbits = (unsigned*)(ws + p.xf_off);
     launch_trig(angles, nv, (double*)(ws + p.trig_off), s, maxbits);
-    if ((flags & NEFCT_F_ADJ_WINDOW) && !L.fan) {
-        // ray tiles with LDS slab windows flushed by global atomics (rays on
-        // fan planes take the float variant of their own adjoint instead)
+    if (flags & NEFCT_F_ADJ_WINDOW) {
+        // ray tiles with LDS slab windows flushed by global atomics
         launch_zero((float*)(ws + p.xf_off), p.xf_elems, s);
         launch_zero((float*)(ws + p.yf_off), p.yf_elems, s);
         const dim3 g((na + BX - 1) / BX, (nb + BY * AR - 1) / (BY * AR), nv), b(BX, BY);
@@ -1939,7 +1959,7 @@ void launch_adjoint_tiles(Launch& L, const float* pv, float* image, unsigned* ma
     const unsigned flags = L.flags;
     const bool ref = (flags & NEFCT_F_REF_SLAB) != 0;
     {
-        const bool fix = !(flags & (NEFCT_F_ADJ_FLOAT_ATOMIC | NEFCT_F_ADJ_WINDOW));
+        const bool fix = !(flags & NEFCT_F_ADJ_FLOAT_ATOMIC);
         // a split of the views adds up in 8 bytes of scratch per voxel
         const size_t nvox = (size_t)L.V.n[0] * L.V.n[1] * L.V.n[2], vol = align256(sizeof(unsigned long long) * nvox);
         const unsigned shape = flags & NEFCT_F_TILE_MASK;
@@ -2002,21 +2022,8 @@ __device__ Launch launch_of(const nefct_problem& pr, char* ws_base, unsigned fla
 {
     Launch L;
     L.zoff = nullptr;
-    for (int i = 0; i < 3; ++i) {
-        L.V.n[i] = pr.grid[i];
-        L.V.vs[i] = (double)pr.size[i] / pr.grid[i];
-        L.V.inv_vs[i] = 1.0 / L.V.vs[i];
-        L.V.lo[i] = (double)pr.center[i] - (double)pr.size[i] * 0.5;
-    }
-    L.G.cyl = pr.cyl;
-    L.G.sid = pr.SID;
-    L.G.sad = pr.SAD;
-    L.G.na = pr.na;
-    L.G.nb = pr.nb;
-    L.G.da = pr.da;
-    L.G.ai = pr.ai;
-    L.G.db = pr.db;
-    L.G.bi = pr.bi;
+    geometry_of(pr.grid, pr.center, pr.size, pr.SID, pr.SAD, pr.na, pr.da, pr.ai, pr.nb, pr.db, pr.bi, pr.cyl, L.V,
+                L.G);
     const WsPlan p = plan_ws(pr.grid, pr.nv);
     char* ws = ws_base + pr.ws_offset;
     L.Ly.xf = (float*)(ws + p.xf_off);
@@ -2030,7 +2037,7 @@ __device__ Launch launch_of(const nefct_problem& pr, char* ws_base, unsigned fla
     L.nv = pr.nv;
     L.flags = flags;
     L.sbound = scale_bound(L.V, L.G, flags);
-    L.fan = fan_ok(L.V, L.G, flags) ? 1 : 0;
+    L.fan = 0;      // (the problem's plan says it)
     L.cols = nullptr;
     return L;
 }
@@ -2287,7 +2294,7 @@ int run_adjoint_noalloc(const float* pv, const int grid[3], const float center[3
     p.trig_off = NOALLOC_TRIG_OFF;
     p.xf_off = p.yf_off = 0;
     p.xf_elems = p.yf_elems = 0;
-    Launch L = make_launch(grid, center, size, nv, SID, SAD, na, da, ai, nb, db, bi, cyl, flags, sc, p);
+    Launch L = make_launch(grid, center, size, nv, SID, SAD, na, da, ai, nb, db, bi, cyl, flags, sc, p, true);
     hipStream_t s = (hipStream_t)stream;
     launch_trig(angles, nv, (double*)(sc + NOALLOC_TRIG_OFF), s, (unsigned*)sc);
     launch_adjoint_tiles(L, pv, image, (unsigned*)sc, nullptr, 0, s);
@@ -2396,7 +2403,7 @@ int nefct_siddon_count(const int grid[3], const float center[3], const float siz
     if (!workspace || workspace_bytes < p.total) return NEFCT_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
     char* ws = (char*)workspace;
-    Launch L = make_launch(grid, center, size, nv, SID, SAD, na, da, ai, nb, db, bi, cyl, flags, ws, p);
+    Launch L = make_launch(grid, center, size, nv, SID, SAD, na, da, ai, nb, db, bi, cyl, flags, ws, p, false);
     launch_trig(angles, nv, (double*)(ws + p.trig_off), s);
     if (flags & NEFCT_F_REF_SLAB)
         launch_siddon<2, true>(L, nullptr, nullptr, counts, s);
@@ -2406,22 +2413,25 @@ int nefct_siddon_count(const int grid[3], const float center[3], const float siz
     return NEFCT_OK;
 }
 
+int nefct_siddon_walk(const int grid[3], const float center[3], const float size[3], int nv, float SID, float SAD,
+                      int na, float da, float ai, int nb, float db, float bi, int cyl, unsigned flags, int adjoint)
+{
+    const int st = validate(grid, center, size, /* no angle is read */ size, nv, SID, SAD, na, da, nb, db, ai, bi, flags);
+    if (st) return st;
+    VolDev V;
+    DetDev G;
+    geometry_of(grid, center, size, SID, SAD, na, da, ai, nb, db, bi, cyl, V, G);
+    return walks_fan_planes(V, G, flags, adjoint != 0) ? 1 : 0;
+}
+
 // Whether a problem's rays are walked on fan planes (its tasks are counted accordingly).
+// (The batched adjoint takes none of the plain one's summing variants.)
 static bool plan_is_fan(const nefct_problem& pr, unsigned flags)
 {
     VolDev V;
     DetDev G;
-    for (int i = 0; i < 3; ++i) {
-        V.n[i] = pr.grid[i];
-        V.vs[i] = (double)pr.size[i] / pr.grid[i];
-        V.inv_vs[i] = 1.0 / V.vs[i];
-    }
-    G.sad = pr.SAD;
-    G.na = pr.na;
-    G.nb = pr.nb;
-    G.db = pr.db;
-    G.bi = pr.bi;
-    return fan_ok(V, G, flags);
+    geometry_of(pr.grid, pr.center, pr.size, pr.SID, pr.SAD, pr.na, pr.da, pr.ai, pr.nb, pr.db, pr.bi, pr.cyl, V, G);
+    return walks_fan_planes(V, G, flags, false);
 }
 
 // How the batch was planned, against the flags of this call.

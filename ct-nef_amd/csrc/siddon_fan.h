@@ -857,12 +857,9 @@ void launch_fan_adj(const Launch& L, const float* pv, float* image, unsigned lon
 {
     const int nbz = fan_zblocks(L.V.n[2], FAN_TZ);
     const dim3 g((L.V.n[0] + FB - 1) / FB, (L.V.n[1] + FB - 1) / FB, nbz * nsplit);
-    if (L.flags & (NEFCT_F_ADJ_FLOAT_ATOMIC | NEFCT_F_ADJ_WINDOW)) {
-        if (L.flags & NEFCT_F_DETERMINISTIC)    // one wavefront: float sums in a fixed order
-            hipLaunchKernelGGL((k_fan_adj<false, FAN_TZ, 1>), g, dim3(64), 0, s, L, pv, image, nullptr, 1, maxbits);
-        else
-            hipLaunchKernelGGL((k_fan_adj<false, FAN_TZ, FAN_NW>), g, dim3(64 * FAN_NW), 0, s, L, pv, image, nullptr,
-                               1, maxbits);
+    if (L.flags & NEFCT_F_ADJ_FLOAT_ATOMIC) {
+        hipLaunchKernelGGL((k_fan_adj<false, FAN_TZ, FAN_NW>), g, dim3(64 * FAN_NW), 0, s, L, pv, image, nullptr, 1,
+                           maxbits);
         return;
     }
     hipLaunchKernelGGL((k_fan_adj<true, FAN_TZ, FAN_NW>), g, dim3(64 * FAN_NW), 0, s, L, pv, image,

@@ -57,6 +57,7 @@ _sz = ctypes.c_size_t
 SIGNATURES = {
     "nefct_status_string": [_i],
     "nefct_siddon_workspace_size": [_vp, _i],
+    "nefct_siddon_walk": [_vp, _vp, _vp, _i, _f, _f, _i, _f, _f, _i, _f, _f, _i, _u, _i],
     "nefct_project_flat": [_vp, _vp, _vp, _vp, _vp, _i, _f, _f, _i, _f, _f, _i, _f, _f, _vp, _u, _vp, _sz, _vp],
     "nefct_project_cyli": [_vp, _vp, _vp, _vp, _vp, _i, _f, _f, _i, _f, _f, _i, _f, _f, _vp, _u, _vp, _sz, _vp],
     "nefct_backproject_flat": [_vp, _vp, _vp, _vp, _vp, _i, _f, _f, _i, _f, _f, _i, _f, _f, _vp, _u, _vp, _sz, _vp],

@@ -66,9 +66,10 @@ typedef enum {
  *                             float atomics
  * A non-finite projection value makes the fixed-point result NaN.
  * The exact rule on geometries whose rays step at most one z cell per slab has
- * kernels of its own, whose blocks and ray tiles are fixed: there the shape,
- * lane spacing and forward tile bits below change nothing, and ADJ_WINDOW
- * means FLOAT_ATOMIC. */
+ * kernels of its own (nefct_siddon_walk tells), whose blocks and ray tiles are
+ * fixed: there the shape, lane spacing and forward tile bits below change
+ * nothing.  ADJ_WINDOW, and FLOAT_ATOMIC with DETERMINISTIC, name kernels that
+ * these geometries keep. */
 #define NEFCT_F_DETERMINISTIC 16u
 #define NEFCT_F_ADJ_WINDOW 32u
 #define NEFCT_F_ADJ_FLOAT_ATOMIC 0x1000u
@@ -110,6 +111,13 @@ const char* nefct_status_string(int status);
  * view count (padded volume copies + per-view table).  Replaces the
  * reference's implicit TF allocations; no reference counterpart. */
 size_t nefct_siddon_workspace_size(const int grid[3], int nv);
+
+/* Which kernels a Siddon call of this geometry takes: 1 those of the detector
+ * columns' common in-plane paths, 0 those that walk every ray by itself, or a
+ * negative status.  The flags' launch shapes apply to the latter only.  adjoint:
+ * 0 for the forward.  Host code; no GPU is needed. */
+int nefct_siddon_walk(const int grid[3], const float center[3], const float size[3], int nv, float SID, float SAD,
+                      int na, float da, float ai, int nb, float db, float bi, int cyl, unsigned flags, int adjoint);
 
 /* Forward projection, flat detector.
  * Replaces ProjectFlatOp::Compute (siddon.cc:129-157) + project_flat
