@@ -32,20 +32,19 @@ constexpr int FAN_ZPAD = 2;     // zero border of the z-fastest copy's rows
 // in-plane step in voxels), slabs [s0, s1) inside the box (none when it
 // misses), the transverse coordinate a(t) = Aa + ka t at slab face t; and what
 // its rays have in common: kz = b dk cells per slab and, above the view's
-// z0, Zc = b dz cells at the end tz towards the source for detector height b
-// (mm).  (From b itself, which is exactly 0 in a middle row: its ray stays in the source's
+// z0, Zc = b dz cells at the slab tz for detector height b (mm).  (From b itself, which is exactly 0 in a middle row: its ray stays in the source's
 // plane.)  One record per column and view is worked out once per call where
 // the workspace has room: the adjoint reads it in every block it passes.
 struct __align__(16) FanCol {
     double ka, ika, Aa, dk, dz;
     double l2;       // squared in-plane source-detector distance in x voxels (1/L^2 scale)
     double p2;       // squared in-plane mm per slab
-    unsigned slabs;  // s0, s1 (15 bits each: grid sides are at most 16384), walk axis (bit 30), path against it (31)
+    unsigned slabs;  // s0, s1 (15 bits each: grid sides are at most 16384), walk axis (bit 30)
+    int tz;          // origin of z along the path (see FanRay)
     __device__ int s0() const { return slabs & 0x7fff; }
     __device__ int s1() const { return (slabs >> 15) & 0x7fff; }
-    __device__ int m() const { return (slabs >> 30) & 1; }
+    __device__ int m() const { return slabs >> 30; }
     __device__ int tc() const { return (s0() + s1()) >> 1; }        // middle slab
-    __device__ int tz() const { return slabs >> 31 ? s1() : s0(); } // the end towards the source
 };
 static_assert(sizeof(FanCol) == 64, "read as four 16-byte words");
 
@@ -90,9 +89,11 @@ __device__ __forceinline__ FanCol fan_column(const VolDev& V, const DetDev& G, d
     const bool hit = dm != 0.0 && tout > tin;
     const int s0 = max((int)floor(tin), 0), s1 = min((int)ceil(tout), nm);
     const int b = hit ? s0 : 0, e = hit && s1 > s0 ? s1 : b;
-    C.slabs = (unsigned)b | (unsigned)e << 15 | (x ? 0u : 1u << 30) | (dm < 0.0 ? 1u << 31 : 0u);
+    C.slabs = (unsigned)b | (unsigned)e << 15 | (x ? 0u : 1u << 30);
+    const int near = dm > 0.0 ? b : e;      // the path's end towards the source
+    C.tz = fabs((double)C.tc() - um) > 2.0 * fabs((double)near - um) ? near : C.tc();
     C.dk = V.inv_vs[2] * idm;
-    C.dz = C.dk * ((double)C.tz() - um);
+    C.dz = C.dk * ((double)C.tz - um);
     const double kt = C.ka * vt;
     C.p2 = fma(kt, kt, vm * vm);
     const double x0 = e0 * V.inv_vs[0], x1 = e1 * V.inv_vs[0];
@@ -110,15 +111,16 @@ __device__ __forceinline__ double fan_z0(const VolDev& V, double lift)
 // z of a ray over its column's path: z(t) = kz (t - tz) + Zc, in cells from
 // the volume's middle cell (nz / 2); ink = 1 / |kz| (capped: a level ray
 // never reaches the next cell); scale = mm per slab.
-// The origin tz is the path's end towards the source.  A ray that meets the
-// volume at all is between the source's height and its own there, so |Zc| stays
-// within the volume (for a source inside its height) and z carries the rounding
-// of numbers of the volume's size, as in the per-ray walk's coordinate about
-// the ray's own middle.  About the path's middle, where a steep ray is far
-// outside, it was up to 3.5 times that (256 x 256 x 16 voxels, source 62 voxels
-// from the volume's face, slopes above 0.2: 1.4e-6 cells rms, now and in the
-// per-ray walk 4.0e-7).  Slope, reciprocal and length per slab are rounded
-// once, from FP64.
+// z carries the rounding of numbers of the size of Zc.  The origin tz is the
+// middle of the column's path, or its end towards the source where the middle
+// is more than twice as far from the source as that: a steep ray that meets the
+// volume near the source is far outside it at the middle, while at the near
+// end it is between the source's height and its own.  (The per-ray walk takes
+// the middle of each ray's own path.  256 x 256 x 16 voxels, source 62 voxels
+// from the volume's face, slopes above 0.2: 4.0e-7 cells rms, about the middle
+// 1.4e-6, per ray 4.1e-7; up to a factor of two, as in usual scans, the middle
+// costs 1 to 12 %.)  Slope, reciprocal and length per slab are rounded once,
+// from FP64.
 struct FanRay {
     float kz, Zc, ink, scale;
 };
@@ -206,7 +208,7 @@ __device__ __forceinline__ FanSlab fan_slab(const FanCol& C, int t, int ha)
         s.d0 = cross ? cross_frac(cell_frac(a0), ika, ka > 0.0f ? ika : 0.0f) : 1.0f;
         s.d1 = 1.0f - s.d0;
     }
-    s.ts = (float)(t - C.tz());
+    s.ts = (float)(t - C.tz);
     const bool in = t >= C.s0() && t < C.s1();
     const bool parts = cross && fan_slow(C);    // both, whatever the column's own lengths
     s.v0 = in && (parts || s.d0 > 0.0f);
@@ -225,12 +227,12 @@ __device__ __forceinline__ FanOwn fan_own(const VolDev& V, const DetDev& G, cons
     FanOwn w;
     const double b = fma(G.bi + ib, G.db, -(G.nb * G.db * 0.5));
     const double kz = b * C.dk, uz = z0 + (double)(V.n[2] >> 1);
-    const double A = fma(b, fma(-C.dk, (double)C.tz(), C.dz), uz);      // z at slab face 0
+    const double A = fma(b, fma(-C.dk, (double)C.tz, C.dz), uz);      // z at slab face 0
     double tin = 0.0, tout = 16384.0;
     clip_axis(kz, kz != 0.0 ? rcp64(kz) : 0.0, A, 0.0, (double)V.n[2], tin, tout);
     const int s0 = max(C.s0(), (int)floor(fmin(tin, 16384.0))), s1 = min(C.s1(), (int)ceil(fmax(tout, 0.0)));
     const int tc = (s0 + s1) >> 1;
-    w.shift = (float)(tc - C.tz());
+    w.shift = (float)(tc - C.tz);
     w.Ac = (float)(fma(C.ka, (double)tc, C.Aa) - ha);
     w.ka = (float)C.ka;
     w.ika = (float)C.ika;
@@ -426,7 +428,7 @@ __device__ __forceinline__ void fan_forward_wave(const Launch& P, int ia, int ib
     float kz = q.kz, Zc = q.Zc, ink = q.ink;
     float lo = 3.0e38f, hi = -3.0e38f;      // slabs (from tz) that some ray spends inside the volume
     bool rests = false;
-    const float e0 = (float)(C.s0() - C.tz()), e1 = (float)(C.s1() - C.tz());
+    const float e0 = (float)(C.s0() - C.tz), e1 = (float)(C.s1() - C.tz);
     const float zlo = (float)(-hz) - 0.0625f, zhi = (float)(nz - hz) + 0.0625f;
     {
         const float za = fmaf(kz, e0, Zc), zb = fmaf(kz, e1, Zc);
@@ -456,9 +458,9 @@ __device__ __forceinline__ void fan_forward_wave(const Launch& P, int ia, int ib
     hi = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, hi)));
     float acc = 0.0f;
     if (lo < hi) {
-        const int t0 = __builtin_amdgcn_readfirstlane(max(C.s0(), C.tz() + (int)floorf(lo)));
-        const int t1 = __builtin_amdgcn_readfirstlane(min(C.s1(), C.tz() + (int)ceilf(hi)));
-        const float w0 = (float)(t0 - C.tz()), w1 = (float)(t1 - C.tz());
+        const int t0 = __builtin_amdgcn_readfirstlane(max(C.s0(), C.tz + (int)floorf(lo)));
+        const int t1 = __builtin_amdgcn_readfirstlane(min(C.s1(), C.tz + (int)ceilf(hi)));
+        const float w0 = (float)(t0 - C.tz), w1 = (float)(t1 - C.tz);
         const float za = fmaf(kz, w0, Zc), zb = fmaf(kz, w1, Zc);
         // no ray's two cells leave -2 .. nz + 1 over [t0, t1]: no clamp
         const float down = kz < 0.0f ? 1.0f : 0.0f;
