@@ -19,9 +19,10 @@
 //    copy, so an index error reads 0 / drops the atomic instead of faulting;
 //  * the adjoint scatters with buffer float atomics into the same two
 //    layouts, then one pass sums them into the x-fastest output.
-// The exact pair of every geometry without steep rays takes the fan-plane
-// kernels of siddon_fan.h instead; the walks here take the reference rule,
-// the counter and steep rays.
+// The exact pair of most geometries without steep rays takes the fan-plane
+// kernels of siddon_fan.h instead (walks_fan_planes); the walks here take the
+// reference rule, the counter, steep rays, detectors of few or distant rows and
+// two of the adjoint's summing variants.
 #include <algorithm>
 #include <type_traits>
 #include <cmath>
@@ -1815,17 +1816,82 @@ __host__ __device__ inline void geometry_of(const int grid[3], const float cente
     G.bi = bi;
 }
 
+// Detector rows between the volume's top and bottom, seen at the axis, in how
+// many of the forward's 64-row tiles, and the pitches of columns (a) and rows
+// (b) there in voxels.  (A helical lift is on the device and not looked at.)
+struct ScanShape {
+    double rows, tiles, pa, pb;
+};
+
+ScanShape scan_shape(const VolDev& V, const DetDev& G)
+{
+    ScanShape c;
+    const double mag = G.sad / G.sid;
+    c.pa = (G.cyl ? G.da * G.sad : G.da) / mag * 0.5 * (V.inv_vs[0] + V.inv_vs[1]);
+    c.pb = G.db / mag * V.inv_vs[2];
+    const double row0 = 0.5 * G.nb - G.bi + 0.5;
+    const double lo = std::max(0.0, V.lo[2] * mag / G.db + row0);
+    const double hi = std::min((double)G.nb, (V.lo[2] + V.n[2] * V.vs[2]) * mag / G.db + row0);
+    c.rows = std::max(1.0, hi - lo);
+    c.tiles = hi > lo ? std::max(1.0, std::ceil(hi / 64 - 1e-6) - std::floor(lo / 64 + 1e-6)) : 1.0;
+    return c;
+}
+
+// Whether the forward is faster on fan planes.  There a wavefront is 64 rows of
+// one column: few rows leave its lanes idle, and rows further apart than a
+// voxel spread its two gathers over more cache lines (per wavefront of a
+// 318-slab path 7.1 ns at half a voxel, 11.1 at one, 19.7 at 1.4, 29 at 4).  The
+// per-ray walk's wavefronts of 16 columns x 4 rows do not mind the rows and like
+// fine columns (8.1 ns at half a voxel, 12.5 at one, 16.3 at 1.6), but copy the
+// volume twice.  The two times in us below, with the latency of a path where
+// the chip is not full, were fitted to 1164 scans (sides 48 to 512, 1 to 300
+// rows, 8 to 360 views, row pitches 0.3 to 7, column pitches 0.3 to 1.7 voxels):
+// the chosen walk takes 2 % more than the faster one on average and at most 1.5
+// times as much; always fan planes took 1.3 times on average and up to 9.6 times
+// as much (512 x 512 x 8, 150 views of 1024 x 8 cells: 1768 against 588 us).
+bool fan_forward_pays(const VolDev& V, const DetDev& G, int nv)
+{
+    const ScanShape c = scan_shape(V, G);
+    const double side = std::max(V.n[0], V.n[1]), walk = (double)nv * G.na * side;
+    const double mvox = 1e-6 * V.n[0] * V.n[1] * (V.n[2] + 4.0);
+    const double spread = c.pb + 2.4 * std::min(std::max((c.pb - 1.0) / 0.3, 0.0), 1.0) +
+                          0.26 * std::max(c.pb - 1.3, 0.0);
+    const double fan = 15.0 + 4.0 * mvox +
+                       std::hypot(walk * (22.3e-6 * c.tiles + 16.7e-6 * c.rows / 64.0 * spread), 0.15 * side);
+    const double ray = 26.0 + 9.0 * mvox +
+                       std::hypot(walk * 24.5e-6 * std::ceil(c.rows / 4.0) / 16.0 * (1.0 + c.pa), 0.23 * side);
+    return fan < ray;
+}
+
+// Whether the adjoint is faster on fan planes.  Its wavefronts deal 16 rows of
+// each of four columns: with few rows (fewer still where columns are coarse, of
+// which the per-ray walk's wavefronts then hold fewer) most lanes idle, and the
+// per-ray blocks win where they fill the chip.  180 views, columns half a voxel
+// apart, us per ray / on fan planes: 512 x 512 x 4 908 / 2250, x 16 1590 / 2191,
+// x 20 2539 / 3143 (x 32, 150 views: 2635 / 2714); 320 x 320 x 4, 100 blocks,
+// 397 / 1045, and without a split of the views, as in a batch, 977; 288 x 288 x
+// 4, 81 blocks, unsplit 962 / 899.  In taller volumes the per-ray blocks, 16
+// voxels high, see no more rows than the fan planes' 52 (256 x 256 x 128, 60
+// views of 512 x 8 cells: 640 / 565).
+bool fan_adjoint_pays(const VolDev& V, const DetDev& G)
+{
+    const ScanShape c = scan_shape(V, G);
+    const double blocks = std::ceil(V.n[0] / 32.0) * std::ceil(V.n[1] / 32.0) * std::ceil(V.n[2] / 16.0);
+    return c.rows * std::max(1.0, c.pa / 0.4) >= 31.0 || blocks < 80.0 || V.n[2] > 32;
+}
+
 // Whether a call's rays are walked on fan planes (siddon_fan.h) or each by its
 // own lane.  Of the adjoint's variants the slab windows and the float sums in a
 // fixed order keep the per-ray kernels: on fan planes they would be the float
 // atomics' blocks, 64^3 voxels, 60 views of 128^2 cells in 3305 us against 538
 // (windows), and the same blocks with one wavefront each, 5239 against 1788 us.
-bool walks_fan_planes(const VolDev& V, const DetDev& G, unsigned flags, bool adjoint)
+bool walks_fan_planes(const VolDev& V, const DetDev& G, int nv, unsigned flags, bool adjoint)
 {
     if (!fan_ok(V, G, flags)) return false;
+    if (!adjoint) return fan_forward_pays(V, G, nv);
     const unsigned ordered = NEFCT_F_ADJ_FLOAT_ATOMIC | NEFCT_F_DETERMINISTIC;
-    if (adjoint && ((flags & NEFCT_F_ADJ_WINDOW) || (flags & ordered) == ordered)) return false;
-    return true;
+    if ((flags & NEFCT_F_ADJ_WINDOW) || (flags & ordered) == ordered) return false;
+    return fan_adjoint_pays(V, G);
 }
 
 Launch make_launch(const int grid[3], const float center[3], const float size[3], int nv, float SID, float SAD,
@@ -1846,7 +1912,7 @@ Launch make_launch(const int grid[3], const float center[3], const float size[3]
     L.nv = nv;
     L.flags = flags;
     L.sbound = scale_bound(L.V, L.G, flags);
-    L.fan = walks_fan_planes(L.V, L.G, flags, adjoint) ? 1 : 0;
+    L.fan = walks_fan_planes(L.V, L.G, nv, flags, adjoint) ? 1 : 0;
     L.cols = nullptr;
     return L;
 }
@@ -2015,6 +2081,13 @@ void launch_adjoint_tiles(Launch& L, const float* pv, float* image, unsigned* ma
 // ---------------------------------------------------------------------------
 // Batched problems (one launch per direction over the tasks of every problem)
 // ---------------------------------------------------------------------------
+// A problem's walks, in its pad_: 0 per ray, 1 on fan planes, FAN_FORWARD or
+// FAN_ADJOINT on fan planes in that direction only.
+constexpr int FAN_FORWARD = 2, FAN_ADJOINT = 3;
+__host__ __device__ inline bool fan_problem(const nefct_problem& pr, int direction)
+{
+    return pr.pad_ == 1 || pr.pad_ == direction;
+}
 constexpr int BTX = 32, BTY = 32, BTZ = 16, BNW = 16;  // adjoint block: the plain default
 constexpr int Q_HEADER = 256;            // workspace head (reserved), then one Launch per problem
 
@@ -2066,10 +2139,10 @@ __host__ __device__ inline size_t batch_max_off(int nprob) { return Q_HEADER + b
 __host__ __device__ inline size_t batch_head_bytes(int nprob) { return batch_max_off(nprob) + align256(4 * (size_t)nprob); }
 
 // trig tables and launch parameters of every problem; zeroed max words
-// cols: 1 in a forward (the column records follow the volume's copy), 2 in an
-// adjoint (they take its place)
+// (in a forward the column records follow the volume's copy, in an adjoint they
+// take its place)
 __global__ void k_batch_prep(const nefct_problem* __restrict__ probs, int nprob, char* ws_base, unsigned flags,
-                             int cols)
+                             int direction)
 {
     const int p = blockIdx.y;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2077,9 +2150,9 @@ __global__ void k_batch_prep(const nefct_problem* __restrict__ probs, int nprob,
     const nefct_problem& pr = probs[p];
     if (i == 0) {
         Launch L = launch_of(pr, ws_base, flags);
-        if (pr.pad_) {
+        if (fan_problem(pr, direction)) {
             const WsPlan w = plan_ws(pr.grid, pr.nv);
-            const size_t off = w.xf_off + (cols == 1 ? align256(sizeof(float) * (size_t)pr.grid[0] * pr.grid[1] *
+            const size_t off = w.xf_off + (direction == FAN_FORWARD ? align256(sizeof(float) * (size_t)pr.grid[0] * pr.grid[1] *
                                                                 fan_row(pr.grid[2])) : 0);
             if (off + sizeof(FanCol) * (size_t)pr.na * (size_t)pr.nv <= w.total) L.cols = ws_base + pr.ws_offset + off;
         }
@@ -2121,7 +2194,7 @@ __device__ __forceinline__ void batch_fwd_task(const nefct_problem* __restrict__
 // eighth of its tasks: all XCDs work on the same problem at a time (one
 // volume in the shared cache, as in one plain call), each on its own views.
 // t0 (a multiple of 8) offsets the chunk this launch covers.
-// Problems walked on fan planes (pad_ = 1) are k_batch_fan_fwd's: their tiles
+// Problems walked on fan planes are k_batch_fan_fwd's: their tiles
 // are counted by its own tile size.
 template <bool REF>
 __global__ __launch_bounds__(FX * FY) void k_batch_fwd(const nefct_problem* __restrict__ probs, int nprob,
@@ -2131,7 +2204,7 @@ __global__ __launch_bounds__(FX * FY) void k_batch_fwd(const nefct_problem* __re
     if (id >= total) return;
     const int p = __builtin_amdgcn_readfirstlane(find_problem(probs, nprob, id, false));
     const nefct_problem& pr = probs[p];
-    if (pr.pad_) return;
+    if (fan_problem(pr, FAN_FORWARD)) return;
     int iv, ta, tb;
     batch_fwd_task(probs, nprob, p, id, total, iv, ta, tb);
     if (iv >= pr.nv) return;
@@ -2148,7 +2221,7 @@ __global__ __launch_bounds__(64 * FAN_FW, 8) void k_batch_fan_fwd(const nefct_pr
     if (id >= total) return;
     const int p = __builtin_amdgcn_readfirstlane(find_problem(probs, nprob, id, false));
     const nefct_problem& pr = probs[p];
-    if (!pr.pad_) return;
+    if (!fan_problem(pr, FAN_FORWARD)) return;
     int iv, ta, tb;
     batch_fwd_task(probs, nprob, p, id, total, iv, ta, tb);
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -2197,7 +2270,7 @@ __global__ __launch_bounds__(64 * BNW) void k_batch_adj(const nefct_problem* __r
     if (t >= total) return;
     const int p = __builtin_amdgcn_readfirstlane(find_problem(probs, nprob, t, true));
     const nefct_problem& pr = probs[p];
-    if (pr.pad_) return;        // k_batch_fan_adj's
+    if (fan_problem(pr, FAN_ADJOINT)) return;       // k_batch_fan_adj's
     // block coordinates made scalar: in vector registers they would carry the
     // block bounds and their derived values into VGPRs
     const int local = __builtin_amdgcn_readfirstlane((int)(t - pr.block_begin));
@@ -2222,7 +2295,7 @@ __global__ __launch_bounds__(64 * FAN_NW, 4) void k_batch_fan_adj(const nefct_pr
     if (t >= total) return;
     const int p = __builtin_amdgcn_readfirstlane(find_problem(probs, nprob, t, true));
     const nefct_problem& pr = probs[p];
-    if (!pr.pad_) return;
+    if (!fan_problem(pr, FAN_ADJOINT)) return;
     const int local = __builtin_amdgcn_readfirstlane((int)(t - pr.block_begin));
     const int bx = __builtin_amdgcn_readfirstlane(local % pr.blocks[0]);
     const int by = __builtin_amdgcn_readfirstlane((local / pr.blocks[0]) % pr.blocks[1]);
@@ -2421,30 +2494,35 @@ int nefct_siddon_walk(const int grid[3], const float center[3], const float size
     VolDev V;
     DetDev G;
     geometry_of(grid, center, size, SID, SAD, na, da, ai, nb, db, bi, cyl, V, G);
-    return walks_fan_planes(V, G, flags, adjoint != 0) ? 1 : 0;
+    return walks_fan_planes(V, G, nv, flags, adjoint != 0) ? 1 : 0;
 }
 
-// Whether a problem's rays are walked on fan planes (its tasks are counted accordingly).
-// (The batched adjoint takes none of the plain one's summing variants.)
-static bool plan_is_fan(const nefct_problem& pr, unsigned flags)
+// A problem's walks (its tasks and blocks are counted accordingly); the batched
+// adjoint takes none of the plain one's summing variants.
+static int plan_walks(const nefct_problem& pr, unsigned flags)
 {
     VolDev V;
     DetDev G;
     geometry_of(pr.grid, pr.center, pr.size, pr.SID, pr.SAD, pr.na, pr.da, pr.ai, pr.nb, pr.db, pr.bi, pr.cyl, V, G);
-    return walks_fan_planes(V, G, flags, false);
+    const unsigned fl = flags & ~(NEFCT_F_ADJ_FLOAT_ATOMIC | NEFCT_F_ADJ_WINDOW | NEFCT_F_DETERMINISTIC);
+    const bool forward = walks_fan_planes(V, G, pr.nv, fl, false), adjoint = walks_fan_planes(V, G, pr.nv, fl, true);
+    return forward && adjoint ? 1 : forward ? FAN_FORWARD : adjoint ? FAN_ADJOINT : 0;
 }
 
-// How the batch was planned, against the flags of this call.
+// How the batch was planned for a direction, against the flags of this call.
 struct BatchKinds {
     bool fan = false, plain = false, mismatch = false;
 };
 
-static BatchKinds batch_kinds(const nefct_problem* host, int nprob, unsigned flags)
+static BatchKinds batch_kinds(const nefct_problem* host, int nprob, unsigned flags, int direction)
 {
     BatchKinds k;
     for (int i = 0; i < nprob; ++i) {
-        (host[i].pad_ ? k.fan : k.plain) = true;
-        if (host[i].pad_ && !plan_is_fan(host[i], flags)) k.mismatch = true;
+        const bool fan = fan_problem(host[i], direction);
+        (fan ? k.fan : k.plain) = true;
+        nefct_problem now = host[i];
+        now.pad_ = plan_walks(now, flags);
+        if (fan && !fan_problem(now, direction)) k.mismatch = true;
     }
     return k;
 }
@@ -2462,12 +2540,13 @@ int nefct_batch_plan(nefct_problem* probs, int nprob, unsigned flags, size_t* wo
                           pr.ai, pr.bi, flags);
         if (st) return st;
         if (!pr.volume || !pr.sinogram) return NEFCT_ERR_NULL;
-        const bool fan = plan_is_fan(pr, flags);
-        pr.pad_ = fan ? 1 : 0;
+        pr.pad_ = plan_walks(pr, flags);
+        bool fan = fan_problem(pr, FAN_FORWARD);
         pr.tiles_a = fan ? (pr.na + FAN_FW - 1) / FAN_FW : (pr.na + FX - 1) / FX;
         pr.tiles_b = fan ? (pr.nb + 63) / 64 : (pr.nb + FY - 1) / FY;
         pr.tile_begin = tiles;
         tiles += (long long)pr.tiles_a * pr.tiles_b * ((pr.nv + FWD_VG - 1) / FWD_VG * FWD_VG);
+        fan = fan_problem(pr, FAN_ADJOINT);
         pr.blocks[0] = fan ? (pr.grid[0] + FB - 1) / FB : (pr.grid[0] + BTX - 1) / BTX;
         pr.blocks[1] = fan ? (pr.grid[1] + FB - 1) / FB : (pr.grid[1] + BTY - 1) / BTY;
         pr.blocks[2] = fan ? fan_zblocks(pr.grid[2], FAN_TZ) : (pr.grid[2] + BTZ - 1) / BTZ;
@@ -2483,11 +2562,12 @@ int nefct_batch_plan(nefct_problem* probs, int nprob, unsigned flags, size_t* wo
 }
 
 static int batch_prep(const nefct_problem* host, const nefct_problem* dev, int nprob, char* ws, unsigned flags,
-                      int cols, hipStream_t s)
+                      int direction, hipStream_t s)
 {
     int maxnv = 1;
     for (int i = 0; i < nprob; ++i) maxnv = max(maxnv, host[i].nv);
-    hipLaunchKernelGGL(k_batch_prep, dim3((maxnv + 255) / 256, nprob), dim3(256), 0, s, dev, nprob, ws, flags, cols);
+    hipLaunchKernelGGL(k_batch_prep, dim3((maxnv + 255) / 256, nprob), dim3(256), 0, s, dev, nprob, ws, flags,
+                       direction);
     return NEFCT_OK;
 }
 
@@ -2512,7 +2592,7 @@ int nefct_batch_project(const nefct_problem* host, const nefct_problem* dev, int
         return NEFCT_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
     char* ws = (char*)workspace;
-    const BatchKinds kinds = batch_kinds(host, nprob, flags);
+    const BatchKinds kinds = batch_kinds(host, nprob, flags, FAN_FORWARD);
     if (kinds.mismatch) {       // planned for the exact rule, called with the reference's: one by one
         for (int i = 0; i < nprob; ++i) {
             const nefct_problem& q = host[i];
@@ -2523,11 +2603,11 @@ int nefct_batch_project(const nefct_problem* host, const nefct_problem* dev, int
         }
         return NEFCT_OK;
     }
-    batch_prep(host, dev, nprob, ws, flags, 1, s);
+    batch_prep(host, dev, nprob, ws, flags, FAN_FORWARD, s);
     for (int i = 0; i < nprob; ++i) {
         const WsPlan p = plan_ws(host[i].grid, host[i].nv);
         char* w = ws + host[i].ws_offset;
-        if (host[i].pad_)
+        if (fan_problem(host[i], FAN_FORWARD))
             launch_fan_prep(host[i].volume, host[i].grid, (float*)(w + p.xf_off), nullptr, 0, nullptr, s);
         else
             launch_pad(host[i].volume, host[i].grid, p, w, s);
@@ -2562,7 +2642,7 @@ int nefct_batch_backproject(const nefct_problem* host, const nefct_problem* dev,
         return NEFCT_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
     char* ws = (char*)workspace;
-    const BatchKinds kinds = batch_kinds(host, nprob, flags);
+    const BatchKinds kinds = batch_kinds(host, nprob, flags, FAN_ADJOINT);
     if (kinds.mismatch) {
         // (the launch-shape flags that the batch does not know are dropped, as below)
         const unsigned fl = flags & ~(NEFCT_F_ADJ_FLOAT_ATOMIC | NEFCT_F_ADJ_WINDOW | NEFCT_F_DETERMINISTIC);
@@ -2575,7 +2655,7 @@ int nefct_batch_backproject(const nefct_problem* host, const nefct_problem* dev,
         }
         return NEFCT_OK;
     }
-    batch_prep(host, dev, nprob, ws, flags, 2, s);
+    batch_prep(host, dev, nprob, ws, flags, FAN_ADJOINT, s);
     if (kinds.fan) batch_cols(host, nprob, ws, s);
     size_t maxn = 1;
     for (int i = 0; i < nprob; ++i)

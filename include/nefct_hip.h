@@ -218,7 +218,7 @@ typedef struct {
     long long ws_offset;    /* byte offset of the problem's workspace region */
     int tiles_a, tiles_b;
     int blocks[3];
-    int pad_;            /* work mapping chosen by nefct_batch_plan */
+    int pad_;            /* work mappings chosen by nefct_batch_plan */
 } nefct_problem;
 
 /* Validates the problems, fills their plan fields and returns the workspace
