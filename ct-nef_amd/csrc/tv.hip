@@ -70,13 +70,13 @@ __device__ __forceinline__ double block_sum(double v)
     return v;
 }
 
-// grad (may be null) = scale * dTV/dx; *value (may be null) += scale * TV(x).
+// grad (with GRAD) = scale * dTV/dx; *value (with VALUE) += scale * TV(x).
 // A workgroup sums zc planes of its 64 x 4 columns before its one atomic:
 // additions to one FP64 word run one after another (~11 ns each), and one per
 // plane and 256 voxels took longer than the sweep itself (128^3 with
 // 8192 workgroups: 102 us; k_sqnorm of 11.8 M values with 4096: 54 us; a
 // descent step takes 106 us less with both).
-template <bool GRAD>
+template <bool GRAD, bool VALUE>
 __global__ __launch_bounds__(256) void k_tv(const float* __restrict__ x, int nx, int ny, int nz, int zc, float e2,
                                             float scale, float* __restrict__ grad, double* __restrict__ value)
 {
@@ -92,15 +92,16 @@ __global__ __launch_bounds__(256) void k_tv(const float* __restrict__ x, int nx,
                 float val;
                 const float g = tv_grad_at(x, ix, iy, iz, nx, ny, nz, e2, val);
                 grad[o] = scale * g;
-                v += val;
+                if (VALUE) v += val;
             } else {
                 v += tv_value_at(x, o, ix, iy, iz, sy, sz, e2);
             }
         }
     }
-    if (!value) return;
-    v = block_sum<4>(v);
-    if (threadIdx.x == 0) atomicAdd(value, (double)scale * v);
+    if constexpr (VALUE) {
+        v = block_sum<4>(v);
+        if (threadIdx.x == 0) atomicAdd(value, (double)scale * v);
+    }
 }
 
 // *value += scale * sum x^2 (FP64 partial sums, one atomic per workgroup)
@@ -159,16 +160,16 @@ int nefct_tv_smooth(const float* image, const int grid[3], float eps, float scal
     if (st) return st;
     if (!image || (!grad && !value)) return NEFCT_ERR_NULL;
     if (!(eps > 0.0f) || !std::isfinite(eps) || !std::isfinite(scale)) return NEFCT_ERR_GEOMETRY;
-    // about 1024 workgroups (four per CU) where the planes allow it
+    // with a value about 1024 workgroups (four per CU) where the planes allow it;
+    // the gradient alone has no atomics to save and one plane to a workgroup
+    // hides more latency (512 x 512 x 256: 385 us, with 1024 workgroups 700)
     const long long columns = (long long)((grid[0] + 63) / 64) * ((grid[1] + 3) / 4);
-    const int zc = (int)std::max<long long>(1, std::min<long long>(grid[2], columns * grid[2] / 1024));
+    const int zc =
+        value ? (int)std::max<long long>(1, std::min<long long>(grid[2], columns * grid[2] / 1024)) : 1;
     const dim3 g((grid[0] + 63) / 64, (grid[1] + 3) / 4, (grid[2] + zc - 1) / zc);
-    if (grad)
-        hipLaunchKernelGGL(k_tv<true>, g, dim3(256), 0, (hipStream_t)stream, image, grid[0], grid[1], grid[2], zc,
-                           eps * eps, scale, grad, value);
-    else
-        hipLaunchKernelGGL(k_tv<false>, g, dim3(256), 0, (hipStream_t)stream, image, grid[0], grid[1], grid[2], zc,
-                           eps * eps, scale, grad, value);
+    const auto kernel = !value ? k_tv<true, false> : grad ? k_tv<true, true> : k_tv<false, true>;
+    hipLaunchKernelGGL(kernel, g, dim3(256), 0, (hipStream_t)stream, image, grid[0], grid[1], grid[2], zc, eps * eps,
+                       scale, grad, value);
     NEFCT_CHECK_LAUNCH();
     return NEFCT_OK;
 }

@@ -40,3 +40,29 @@ def test_sq_norm_remainders(n, first):
     value = torch.zeros((), dtype=torch.float64, device=DEV)
     _sq_norm_into(x.to(DEV)[first:], value, 0.5)
     assert value.item() == pytest.approx(want, rel=1e-10)    # FP64 sums of exact squares
+
+
+def test_gradient_alone_is_no_slower_than_the_step_that_contains_it():
+    """The descent step reads one volume more than the gradient and computes the
+    same; sharing planes between workgroups, which only the value's sum needs,
+    made the gradient 1.5 times the step."""
+    from nefct_hip.recon import _tv_hip, tv_descent_step
+    x = torch.rand((192, 512, 512), generator=torch.Generator().manual_seed(3)).to(DEV)
+    d = torch.zeros_like(x)
+
+    def us(fn):
+        fn()
+        best = float("inf")
+        for _ in range(5):
+            e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            e[0].record()
+            for _ in range(5):
+                fn()
+            e[1].record()
+            torch.cuda.synchronize()
+            best = min(best, e[0].elapsed_time(e[1]) * 200.0)
+        return best
+
+    grad = us(lambda: _tv_hip(x, 1e-3, 1.0, False, True))
+    step = us(lambda: tv_descent_step(x, d, 1e-3, 0.1, 0.1))
+    assert grad <= 1.25 * step, (grad, step)
