@@ -77,3 +77,22 @@ def test_invert_stops_on_the_right_state(oracle, iters):
     want = oracle.invert_dvf(*m, iters=iters)
     for k in range(3):
         assert np.max(np.abs(inv[k] - want[k])) < 1e-5
+
+
+@pytest.mark.parametrize("boundary", [0, 1])
+@pytest.mark.parametrize("shape", [(4, 11, 17), (3, 9, 64), (3, 10, 130)])
+def test_adjoint_of_rows_on_voxels_between_others(shape, boundary):
+    """Rows whose samples all lie on voxels (displacements of 0, 1 and -2) or
+    have no gradient hand nothing on; the rows around them do."""
+    from nefct_hip.deform import deform_adjoint_op
+    rng = np.random.default_rng(5)
+    m = _field("smooth", shape, rng)
+    g = rng.standard_normal(shape).astype(np.float32)
+    for y, d in ((1, 0.0), (2, 1.0), (5, -2.0), (8, 0.0)):
+        m[:, :, y] = d
+    g[:, 6] = 0.0
+    t = [torch.tensor(a, device=DEV) for a in (g, *m)]
+    got = deform_adjoint_op(*t, boundary).double().cpu().numpy()
+    want, mag = _scatter(g, m, boundary)
+    # FP32 sums of some tens of products: 4e-6 of the summed magnitudes
+    assert np.all(np.abs(got - want) <= 4e-6 * mag + 1e-30)
