@@ -520,8 +520,10 @@ def main():
         adj_flags, arec = autotune.tune_adjoint(vol, det, ang)
         tuned = {"forward": frec["variant"], "adjoint": arec["variant"],
                  "forward_ms_on_sample": frec["ms_on_sample"], "adjoint_ms_on_sample": arec["ms_on_sample"],
-                 "forward_sample_views": frec["sample_views"], "adjoint_sample_views": arec["sample_views"]}
-        log(f"[bench] tuned: forward {frec['variant']}, adjoint {arec['variant']}")
+                 "forward_sample_views": frec["sample_views"], "adjoint_sample_views": arec["sample_views"],
+                 "forward_walk": frec.get("walk"), "adjoint_walk": arec.get("walk")}
+        log(f"[bench] tuned: forward {frec['variant']} ({frec.get('walk')}), "
+            f"adjoint {arec['variant']} ({arec.get('walk')})")
 
     def step():
         e0 = torch.cuda.Event(enable_timing=True)

@@ -10,8 +10,13 @@ work maps onto the chip (include/nefct_hip.h):
   workgroup (a wavefront is the first 64 of them) and the number of
   neighbouring views each XCD walks together (its L2 reuse).
 
-(The exact rule on usual cones has kernels whose shapes are fixed: there the
-candidates time alike.)  Which is fastest depends on the volume, detector and view count, so the
+Scans whose rays are walked on fan planes (``walks_fan_planes``) have kernels of
+fixed shapes: there the candidates that run the same kernel in the same way are
+timed once and share that time (the adjoint's fixed-point shapes; the forward's
+tiles of one view group), and of these the first is kept.  The record's
+``walk`` says which kind ran.
+
+Which is fastest depends on the volume, detector and view count, so the
 tuner times the candidates on a sample of the views (the forward on a
 contiguous run, since its order exploits neighbouring views; the adjoint on
 an even spread) and keeps the winner per (device, direction, geometry, mode)
@@ -123,6 +128,39 @@ def _time_ms(fn, reps: int) -> float:
     return e0.elapsed_time(e1) / reps
 
 
+def walks_fan_planes(vol: VolumeGeometry, det: ConeGeometry, nv: int, flags: int, adjoint: bool) -> bool:
+    """Whether a call's rays are walked on fan planes or each by itself."""
+    walk = _lib.load().nefct_siddon_walk(
+        _lib.int3([int(g) for g in vol.grid]), _lib.float3([float(c) for c in vol.center]),
+        _lib.float3([float(v) for v in vol.size]), int(nv), det.SID, det.SAD, det.na, det.da, det.ai, det.nb, det.db,
+        det.bi, int(det.cyl), int(flags), int(adjoint))
+    _lib.check(min(walk, 0), "siddon_walk")
+    return walk == 1
+
+
+def _time_candidates(vol, det, nv: int, mode_flags: int, cands: Dict[str, int], adjoint: bool, run, reps: int):
+    """ms of every candidate, run(flags); those that run the same kernel alike are timed once."""
+    counts = _lib.F_ADJ_FLOAT_ATOMIC if adjoint else _lib.F_FWD_VG_MASK    # flags that matter on fan planes
+    times: Dict[str, float] = {}
+    timed: Dict[object, float] = {}
+    for name, fl in cands.items():
+        flags = int(mode_flags) | int(fl)
+        kernel = ("fan", flags & counts) if walks_fan_planes(vol, det, nv, flags, adjoint) else flags
+        if kernel not in timed:
+            timed[kernel] = _time_ms(lambda: run(flags), reps)
+        times[name] = timed[kernel]
+    return times
+
+
+def _record(vol, det, nv: int, mode_flags: int, cands: Dict[str, int], times: Dict[str, float], adjoint: bool,
+            sample_views: int) -> dict:
+    best = min(times, key=times.get)
+    flags = int(mode_flags) | int(cands[best])
+    return {"flags": flags, "variant": best, "sample_views": sample_views,
+            "walk": "fan planes" if walks_fan_planes(vol, det, nv, flags, adjoint) else "per ray",
+            "ms_on_sample": {k: round(v, 3) for k, v in times.items()}}
+
+
 def tune_adjoint(vol: VolumeGeometry, det: ConeGeometry, angles, mode_flags: int = 0,
                  candidates: Optional[Dict[str, int]] = None, sample_views: int = 64, reps: int = 2,
                  force: bool = False) -> Tuple[int, dict]:
@@ -144,13 +182,9 @@ def tune_adjoint(vol: VolumeGeometry, det: ConeGeometry, angles, mode_flags: int
     g = torch.Generator(device=dev).manual_seed(0)
     y = torch.rand((sub.numel(), det.nb, det.na), generator=g, device=dev)
     cands = dict(candidates or ADJOINT_CANDIDATES)
-    times = {}
-    for name, fl in cands.items():
-        flags = int(mode_flags) | int(fl)
-        times[name] = _time_ms(lambda: backproject(y, vol, det, sub, flags=flags), reps)
-    best = min(times, key=times.get)
-    rec = {"flags": int(mode_flags) | int(cands[best]), "variant": best, "sample_views": int(sub.numel()),
-           "ms_on_sample": {k: round(v, 3) for k, v in times.items()}}
+    times = _time_candidates(vol, det, sub.numel(), mode_flags, cands, True,
+                             lambda flags: backproject(y, vol, det, sub, flags=flags), reps)
+    rec = _record(vol, det, nv, mode_flags, cands, times, True, int(sub.numel()))
     _store(key, rec)
     return int(rec["flags"]), rec
 
@@ -178,13 +212,9 @@ def tune_forward(vol: VolumeGeometry, det: ConeGeometry, angles, mode_flags: int
     g = torch.Generator(device=dev).manual_seed(0)
     x = torch.rand(vol.shape_zyx, generator=g, device=dev)
     cands = dict(candidates or FORWARD_CANDIDATES)
-    times = {}
-    for name, fl in cands.items():
-        flags = int(mode_flags) | int(fl)
-        times[name] = _time_ms(lambda: project(x, vol, det, sub, flags=flags), reps)
-    best = min(times, key=times.get)
-    rec = {"flags": int(mode_flags) | int(cands[best]), "variant": best, "sample_views": int(sub.numel()),
-           "ms_on_sample": {k: round(v, 3) for k, v in times.items()}}
+    times = _time_candidates(vol, det, sub.numel(), mode_flags, cands, False,
+                             lambda flags: project(x, vol, det, sub, flags=flags), reps)
+    rec = _record(vol, det, nv, mode_flags, cands, times, False, int(sub.numel()))
     _store(key, rec)
     return int(rec["flags"]), rec
 

@@ -1,12 +1,12 @@
 """Batched Siddon pair over many problems of uneven size.
 
-One launch per direction covers every problem: the forward's workgroups are
-tasks of 4 detector columns by 64 rows (one view, neighbouring views dealt to
-the same XCD) and the adjoint's blocks of 16x16 voxel columns (16x16 rays and
-32x32x16 voxels with the reference rule or steep cones), numbered across all problems, so small
-problems do not leave the GPU idle and there is one launch instead of one per
-problem (the reference loops
-in Python over views and phases, nefct/functions/project_t.py:153-159,
+One launch per direction covers every problem (two where some are walked on fan
+planes and some per ray): the forward's workgroups are tasks of 4 detector
+columns by 64 rows (one view, neighbouring views dealt to the same XCD) and the
+adjoint's blocks of 16x16 voxel columns (16x16 rays and 32x32x16 voxels per
+ray), numbered across all problems, so small problems do not leave the GPU idle
+and there is one launch instead of one per problem (the reference loops in
+Python over views and phases, nefct/functions/project_t.py:153-159,
 back_project_t.py:150-156).
 
 ``SiddonBatch`` owns static device buffers (volumes, sinograms, problem table,
@@ -106,10 +106,15 @@ class SiddonBatch:
         """Times the batched adjoint with neighbouring lanes one and two
         detector rows apart (identical results) on the batch's current
         sinograms and keeps the faster for ``backproject``.  Returns the
-        record (ms per call of each)."""
+        record (ms per call of each; ``walk``: where every problem is walked
+        on fan planes there is one spacing, timed once, and stride1 is kept)."""
         base = self.flags & ~_lib.F_LANE_STRIDE2
+        fan = all(p.pad_ in (1, 3) for p in self.host) and not self.flags & _lib.F_REF_SLAB
         times = {}
         for name, fl in (("stride1", base), ("stride2", base | _lib.F_LANE_STRIDE2)):
+            if fan and times:
+                times[name] = times["stride1"]
+                continue
             self.flags = fl
             self.backproject()
             torch.cuda.synchronize(self.device)
@@ -123,7 +128,7 @@ class SiddonBatch:
             times[name] = round(e0.elapsed_time(e1) / reps, 3)
         best = min(times, key=times.get)
         self.flags = base | (_lib.F_LANE_STRIDE2 if best == "stride2" else 0)
-        return {"adjoint": best, "ms": times}
+        return {"adjoint": best, "ms": times, "walk": "fan planes" if fan else "per ray"}
 
     def backproject(self):
         L = _bind()
