@@ -451,9 +451,9 @@ __global__ __launch_bounds__(256) void k_fdk_bp(const float* __restrict__ q, con
 // leaves nothing to run while its waves wait at the per-view barrier).
 //
 // What bounds the default: vector issue (ten instructions per sample, about
-// 14 with the column's projection: busy 88 % of the time) and, close behind,
-// LDS (two ds_read2_b32 per sample from one address, at constant offsets
-// (0, 1) and (SRS, SRS + 1): busy 77 %).  512 x 512 x 256 voxels, 408 views of
+// 14 with the column's projection: 98 % of the issue slots), with LDS behind
+// (two ds_read2_b32 per sample from one address, at constant offsets
+// (0, 1) and (SRS, SRS + 1): 62 % of its cycles).  512 x 512 x 256 voxels, 408 views of
 // 1024 x 768: 14.0 -> 10.8 ms, from
 //   - rows loaded straight into LDS, one dword per lane (13.7 -> 12.5).  Held
 //     in registers under a branch per 16-byte slot, each load first waited for

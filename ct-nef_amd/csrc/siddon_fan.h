@@ -14,16 +14,18 @@
 // for a piece that covers [f0, f0 + dt] of its slab.  About 10 (forward) and
 // 14 (adjoint) vector instructions per in-plane piece and ray, against 22 and
 // 34 per voxel when every lane walks its own three coordinates: 512 x 512 x
-// 256 voxels, 1024 x 768 cells, 720 views, forward 96.9 -> 76.5 ms, adjoint
-// 262.8 -> 175.0 ms.  What bounds them now: the forward's two gathers per
-// piece keep the CU's texture address unit busy 98 % of the time and its vector
-// issue is nearly full as well; the adjoint fills 80 % of its vector issue
-// slots and about as much of its LDS time (two 64-bit additions per piece,
-// 6.4 clocks of the CU each, and half a table read).
-// Forward and adjoint evaluate the same functions below, so the pair stays an
-// exact transpose; the pieces do not depend on the block they are walked
-// from, so the fixed-point adjoint's bits do not depend on how the volume or
-// the views are split.
+// 256 voxels, 1024 x 768 cells, 720 views, forward 97.1 -> 78.6 ms, adjoint
+// 262.4 -> 181.8 ms.  What bounds them now: the forward's two gathers per
+// piece keep the CU's texture address unit busy 97 % of the time and its vector
+// issue is nearly full as well; the adjoint fills 84 % of its vector issue
+// slots and 56 % of its LDS cycles (two 64-bit additions per piece, 6.4 clocks
+// of the CU each, and half a table read).
+// Forward and adjoint evaluate the same functions below, a column by its own
+// rules whichever others a wavefront takes with it, so the pair holds one
+// matrix up to the rounding of a piece; the pieces do not depend on the block
+// they are walked from, so the fixed-point adjoint's bits do not depend on how
+// the volume or the views are split.  (walks_fan_planes may send one direction
+// of a scan to the per-ray walk: then the two differ by a crossing's rounding.)
 #pragma once
 
 constexpr int FAN_ZPAD = 2;     // zero border of the z-fastest copy's rows
