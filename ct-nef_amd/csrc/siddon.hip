@@ -1521,22 +1521,60 @@ __global__ __launch_bounds__(64 * NW, 4) void k_siddon_adj_tile(Launch P, const 
                                                  es);
 }
 
+// Detector rows between the volume's top and bottom, seen at the axis, in how
+// many of the forward's 64-row tiles, and the pitches of columns (a) and rows
+// (b) there in voxels.  (A helical lift is on the device and not looked at.)
+struct ScanShape {
+    double rows, tiles, pa, pb;
+};
+
+ScanShape scan_shape(const VolDev& V, const DetDev& G)
+{
+    ScanShape c;
+    const double mag = G.sad / G.sid;
+    c.pa = (G.cyl ? G.da * G.sad : G.da) / mag * 0.5 * (V.inv_vs[0] + V.inv_vs[1]);
+    c.pb = G.db / mag * V.inv_vs[2];
+    const double row0 = 0.5 * G.nb - G.bi + 0.5;
+    const double lo = std::max(0.0, V.lo[2] * mag / G.db + row0);
+    const double hi = std::min((double)G.nb, (V.lo[2] + V.n[2] * V.vs[2]) * mag / G.db + row0);
+    c.rows = std::max(1.0, hi - lo);
+    c.tiles = hi > lo ? std::max(1.0, std::ceil(hi / 64 - 1e-6) - std::floor(lo / 64 + 1e-6)) : 1.0;
+    return c;
+}
+
+// us of the adjoint for one block (tx x ty x tz voxels) and view, from the rays
+// of its shadow.  On fan planes, by groups of four columns and 16 rows (fitted
+// to 665 scans); per ray, by wavefronts (exact, us per view at 41, 22, 5
+// wavefronts: 23, 9, 5; reference rule, at 41, 25, 20: 53, 34, 27, of which its
+// blocks, who differ more among each other, want the upper end: 85x85x91, 60
+// views 353 us so, by the mean 398).
+double block_view_us(const Launch& L, int tx, int ty, int tz)
+{
+    const ScanShape c = scan_shape(L.V, L.G);
+    const double side = 0.5 * (std::min(tx, L.V.n[0]) + std::min(ty, L.V.n[1]));
+    const double columns = std::min((double)L.G.na, 1.2 * side / c.pa + 2.0);
+    const double rows = std::min(c.rows, (std::min(tz, L.V.n[2]) + 1.0) / c.pb + 1.0);
+    if (L.fan) return 0.2 + std::ceil(columns / 4.0) * (3.2 + 2.1 * std::ceil(rows / 16.0)) / 16.0;
+    const double waves = std::ceil(columns * rows / 64.0);
+    return L.flags & NEFCT_F_REF_SLAB ? std::min(60.0, 4.0 + 3.0 * waves) : 3.5 + 0.4 * waves;
+}
+
 // Number of view ranges a block's work is split into.  A workgroup fills a
 // CU, so few blocks leave CUs idle (32 blocks at 64^3) or a last round nearly
 // empty; the ranges' integer sums are added in the workspace, one more launch
 // and about 5 ps per voxel and range (2.6 M voxels in five ranges: 64 us).  The
-// number with the least of both, view_us being a block's time per view (about
-// 6 us on fan planes; 20 to 60 us of the per-ray walk, whose blocks differ
-// more, so the upper end).  With at least eight (fan planes) or two views to a
-// range instead: 64x64x40, 12 / 100 views of 83x52 cells 82 -> 41 / 77 -> 65 us,
-// 32x32x24, 40 views 134 -> 34 us; per ray 53x53x25, 14 views 240 -> 126 us,
-// 192x192x200, 100 views 5169 -> 4657 us (but 85x85x91, 21 views 285 -> 371).
-inline int tile_splits(const Launch& L, int tx, int ty, int tz, double view_us)
+// number with the least of both.  64x64x40, 12 / 100 views of 83x52 cells 82 ->
+// 41 / 77 -> 65 us, 32x32x24, 40 views 134 -> 34 us; per ray 53x53x25, 14 views
+// 240 -> 126 us, 192x192x200, 100 views 5169 -> 4657 us.  (With one figure for
+// every block and view, 6 us on fan planes and 60 per ray, calls of few rows or
+// views split for nothing: 207x207x1, 16 views of 207 x 3 cells 46 -> 127 us,
+// 270x41x140, 31 views of 81 x 4 cells 46 -> 214.)
+inline int tile_splits(const Launch& L, int tx, int ty, int tz)
 {
     constexpr int CUS = 256;
     const long long blocks = (long long)((L.V.n[0] + tx - 1) / tx) * ((L.V.n[1] + ty - 1) / ty) *
                              ((L.V.n[2] + tz - 1) / tz);
-    const double voxels = (double)L.V.n[0] * L.V.n[1] * L.V.n[2];
+    const double voxels = (double)L.V.n[0] * L.V.n[1] * L.V.n[2], view_us = block_view_us(L, tx, ty, tz);
     int best = 1;
     double least = 0.0;
     for (int ns = 1; ns <= 64 && ns <= L.nv; ++ns) {
@@ -1583,10 +1621,9 @@ void launch_split_sums(const Launch& L, const unsigned long long* sums, const un
 // 1882 -> 1254 us).
 template <int TX, int TY, int TZ, int NW, int CS>
 void launch_tile(bool ref, bool fix, const Launch& L, const float* pv, float* image, unsigned long long* sums,
-                 const unsigned* maxbits, float sbound, hipStream_t s)
+                 int nsplit, const unsigned* maxbits, float sbound, hipStream_t s)
 {
-    const int ns = (fix && NW == 16 && sums) ? tile_splits(L, TX, TY, TZ, 60.0) : 1;
-    if (ns == 1) sums = nullptr;
+    const int ns = sums ? nsplit : 1;
     const dim3 g((L.V.n[0] + TX - 1) / TX, (L.V.n[1] + TY - 1) / TY, (L.V.n[2] + TZ - 1) / TZ * ns);
     const dim3 b(64 * NW);
     if (ref && fix)
@@ -1816,27 +1853,6 @@ __host__ __device__ inline void geometry_of(const int grid[3], const float cente
     G.bi = bi;
 }
 
-// Detector rows between the volume's top and bottom, seen at the axis, in how
-// many of the forward's 64-row tiles, and the pitches of columns (a) and rows
-// (b) there in voxels.  (A helical lift is on the device and not looked at.)
-struct ScanShape {
-    double rows, tiles, pa, pb;
-};
-
-ScanShape scan_shape(const VolDev& V, const DetDev& G)
-{
-    ScanShape c;
-    const double mag = G.sad / G.sid;
-    c.pa = (G.cyl ? G.da * G.sad : G.da) / mag * 0.5 * (V.inv_vs[0] + V.inv_vs[1]);
-    c.pb = G.db / mag * V.inv_vs[2];
-    const double row0 = 0.5 * G.nb - G.bi + 0.5;
-    const double lo = std::max(0.0, V.lo[2] * mag / G.db + row0);
-    const double hi = std::min((double)G.nb, (V.lo[2] + V.n[2] * V.vs[2]) * mag / G.db + row0);
-    c.rows = std::max(1.0, hi - lo);
-    c.tiles = hi > lo ? std::max(1.0, std::ceil(hi / 64 - 1e-6) - std::floor(lo / 64 + 1e-6)) : 1.0;
-    return c;
-}
-
 // Whether the forward is faster on fan planes.  There a wavefront is 64 rows of
 // one column: few rows leave its lanes idle, and rows further apart than a
 // voxel spread its two gathers over more cache lines (per wavefront of a
@@ -1865,19 +1881,21 @@ bool fan_forward_pays(const VolDev& V, const DetDev& G, int nv)
 
 // Whether the adjoint is faster on fan planes.  Its wavefronts deal 16 rows of
 // each of four columns: with few rows (fewer still where columns are coarse, of
-// which the per-ray walk's wavefronts then hold fewer) most lanes idle, and the
-// per-ray blocks win where they fill the chip.  180 views, columns half a voxel
-// apart, us per ray / on fan planes: 512 x 512 x 4 908 / 2250, x 16 1590 / 2191,
-// x 20 2539 / 3143 (x 32, 150 views: 2635 / 2714); 320 x 320 x 4, 100 blocks,
-// 397 / 1045, and without a split of the views, as in a batch, 977; 288 x 288 x
-// 4, 81 blocks, unsplit 962 / 899.  In taller volumes the per-ray blocks, 16
-// voxels high, see no more rows than the fan planes' 52 (256 x 256 x 128, 60
-// views of 512 x 8 cells: 640 / 565).
+// which the per-ray walk's wavefronts then hold fewer) most lanes idle.  180
+// views, columns half a voxel apart, us per ray / on fan planes: 512 x 512 x 4
+// 908 / 2250, x 16 1590 / 2191, x 20 2539 / 3143 (x 32, 150 views: 2635 / 2714).
+// Small volumes (fewer per-ray blocks than a third of the chip's CUs) and those
+// taller than two per-ray blocks gain from the fan planes' blocks down to a
+// handful of rows (288 x 288 x 4, 81 blocks, 962 / 899 without a split of the
+// views, as in a batch; 256 x 256 x 128, 60 views of 512 x 8 cells: 640 / 565).
+// Of 1164 scans 9 take over 5 % longer than per ray before views were split
+// (up to 1.3 times); always on fan planes 105 would (up to 4.1 times).
 bool fan_adjoint_pays(const VolDev& V, const DetDev& G)
 {
     const ScanShape c = scan_shape(V, G);
     const double blocks = std::ceil(V.n[0] / 32.0) * std::ceil(V.n[1] / 32.0) * std::ceil(V.n[2] / 16.0);
-    return c.rows * std::max(1.0, c.pa / 0.4) >= 31.0 || blocks < 80.0 || V.n[2] > 32;
+    const double rows = c.rows * std::max(1.0, c.pa / 0.4);
+    return rows >= 31.0 || (rows >= 6.0 && (blocks < 80.0 || V.n[2] > 32));
 }
 
 // Whether a call's rays are walked on fan planes (siddon_fan.h) or each by its
@@ -2033,10 +2051,10 @@ void launch_adjoint_tiles(Launch& L, const float* pv, float* image, unsigned* ma
         int nsplit = 1;
         if (sums)
             nsplit = L.fan ? tile_splits(L, FB, FB, (L.V.n[2] + fan_zblocks(L.V.n[2], FAN_TZ) - 1) /
-                                                        fan_zblocks(L.V.n[2], FAN_TZ), 6.0)
-                     : shape == NEFCT_F_TILE_64x32x8 ? tile_splits(L, 64, 32, 8, 60.0)
-                     : shape == NEFCT_F_TILE_64x16x16 ? tile_splits(L, 64, 16, 16, 60.0)
-                     : shape == NEFCT_F_TILE_32x32x16 ? tile_splits(L, 32, 32, 16, 60.0) : 1;
+                                                        fan_zblocks(L.V.n[2], FAN_TZ))
+                     : shape == NEFCT_F_TILE_64x32x8 ? tile_splits(L, 64, 32, 8)
+                     : shape == NEFCT_F_TILE_64x16x16 ? tile_splits(L, 64, 16, 16)
+                     : shape == NEFCT_F_TILE_32x32x16 ? tile_splits(L, 32, 32, 16) : 1;
         if (nsplit == 1) sums = nullptr;
         if (L.fan) {
             const size_t used = sums ? vol : 0;
@@ -2055,25 +2073,25 @@ void launch_adjoint_tiles(Launch& L, const float* pv, float* image, unsigned* ma
         const bool cs2 = (flags & NEFCT_F_LANE_STRIDE2) != 0;
         if (!fix && (flags & NEFCT_F_DETERMINISTIC)) {
             // float accumulation in a fixed order: one wavefront per 16x16x8 block
-            launch_tile<16, 16, 8, 1, 1>(ref, false, L, pv, image, sums, maxbits, sb, s);
+            launch_tile<16, 16, 8, 1, 1>(ref, false, L, pv, image, sums, nsplit, maxbits, sb, s);
         } else if (shape == NEFCT_F_TILE_32x16x8) {
-            if (cs2) launch_tile<32, 16, 8, 4, 2>(ref, fix, L, pv, image, sums, maxbits, sb, s);
-            else launch_tile<32, 16, 8, 4, 1>(ref, fix, L, pv, image, sums, maxbits, sb, s);
+            if (cs2) launch_tile<32, 16, 8, 4, 2>(ref, fix, L, pv, image, sums, nsplit, maxbits, sb, s);
+            else launch_tile<32, 16, 8, 4, 1>(ref, fix, L, pv, image, sums, nsplit, maxbits, sb, s);
         } else if (shape == NEFCT_F_TILE_32x32x8) {
-            if (cs2) launch_tile<32, 32, 8, 4, 2>(ref, fix, L, pv, image, sums, maxbits, sb, s);
-            else launch_tile<32, 32, 8, 4, 1>(ref, fix, L, pv, image, sums, maxbits, sb, s);
+            if (cs2) launch_tile<32, 32, 8, 4, 2>(ref, fix, L, pv, image, sums, nsplit, maxbits, sb, s);
+            else launch_tile<32, 32, 8, 4, 1>(ref, fix, L, pv, image, sums, nsplit, maxbits, sb, s);
         } else if (shape == NEFCT_F_TILE_64x32x8) {
-            if (cs2) launch_tile<64, 32, 8, 16, 2>(ref, fix, L, pv, image, sums, maxbits, sb, s);
-            else launch_tile<64, 32, 8, 16, 1>(ref, fix, L, pv, image, sums, maxbits, sb, s);
+            if (cs2) launch_tile<64, 32, 8, 16, 2>(ref, fix, L, pv, image, sums, nsplit, maxbits, sb, s);
+            else launch_tile<64, 32, 8, 16, 1>(ref, fix, L, pv, image, sums, nsplit, maxbits, sb, s);
         } else if (shape == NEFCT_F_TILE_16x16x32) {
-            if (cs2) launch_tile<16, 16, 32, 4, 2>(ref, fix, L, pv, image, sums, maxbits, sb, s);
-            else launch_tile<16, 16, 32, 4, 1>(ref, fix, L, pv, image, sums, maxbits, sb, s);
+            if (cs2) launch_tile<16, 16, 32, 4, 2>(ref, fix, L, pv, image, sums, nsplit, maxbits, sb, s);
+            else launch_tile<16, 16, 32, 4, 1>(ref, fix, L, pv, image, sums, nsplit, maxbits, sb, s);
         } else if (shape == NEFCT_F_TILE_64x16x16) {
-            if (cs2) launch_tile<64, 16, 16, 16, 2>(ref, fix, L, pv, image, sums, maxbits, sb, s);
-            else launch_tile<64, 16, 16, 16, 1>(ref, fix, L, pv, image, sums, maxbits, sb, s);
+            if (cs2) launch_tile<64, 16, 16, 16, 2>(ref, fix, L, pv, image, sums, nsplit, maxbits, sb, s);
+            else launch_tile<64, 16, 16, 16, 1>(ref, fix, L, pv, image, sums, nsplit, maxbits, sb, s);
         } else {
-            if (cs2) launch_tile<32, 32, 16, 16, 2>(ref, fix, L, pv, image, sums, maxbits, sb, s);
-            else launch_tile<32, 32, 16, 16, 1>(ref, fix, L, pv, image, sums, maxbits, sb, s);
+            if (cs2) launch_tile<32, 32, 16, 16, 2>(ref, fix, L, pv, image, sums, nsplit, maxbits, sb, s);
+            else launch_tile<32, 32, 16, 16, 1>(ref, fix, L, pv, image, sums, nsplit, maxbits, sb, s);
         }
     }
 }
